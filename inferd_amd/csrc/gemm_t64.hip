@@ -312,14 +312,17 @@ static GtPlan gemm_t_plan(int M, int N, int K, int Mrows = 0) {
   return pl;
 }
 
-// Prefill shapes that fill at least one round of 256 CUs with 256-row tiles go to k_gemm_t8 (gemm_t8.hip): half the
-// dequant VALU per MFMA.
-static bool use_t8(int M, int N) { return (long)((M + 255) / 256) * ((t64_bands(N) + 7) / 8) >= 256; }
-
 size_t gemm_t_workspace(int M, int N, int K, int mode) {
-  if (!use_t8(M, N) && gemm_sk_applies(M, N, K, mode)) return gemm_sk_workspace(M, N, K, mode);
-  if (use_t8(M, N))
-    return align_up(gemm_t8_workspace(M, N, K), 256) + (mode == kModeSwiglu ? (size_t)M * N * sizeof(uint16_t) : 0);
+  // The size of a prefill shape decides which requests the static scratch of ifd_gemm_t64_noalloc serves, so it is never
+  // less than a split of 256-row tiles (from a round of them) or the stream-K kernel (below) would need.
+  if (gemm_w_applies(M, N, K, mode)) {
+    const long tiles = (long)((M + 255) / 256) * ((t64_bands(N) + 7) / 8), tail = tiles % 256;
+    size_t least = 0;
+    if (tiles < 256) least = gemm_sk_applies(M, N, K, mode) ? gemm_sk_workspace(M, N, K, mode) : 0;
+    else if (tail && tail <= 128) least = (size_t)std::min({256 / tail, 8L, K / kGroup / 4L}) * tail * 256 * 256 * 4;
+    return std::max(gemm_w_workspace(M, N, K), least);
+  }
+  if (gemm_sk_applies(M, N, K, mode)) return gemm_sk_workspace(M, N, K, mode);
   return epilogue_ws_bytes(gemm_t_plan(M, N, K).S, M, N, mode);
 }
 
@@ -368,19 +371,15 @@ int launch_gemm_t(const uint16_t* A, int lda, const void* wt, int N, int K, void
                   void* ws, size_t ws_bytes, hipStream_t st) {
   if (M == 0) return IFD_OK;
   if (K % 128) return fail(IFD_ERR_ARG, "T64 GEMM needs K %% 128 == 0 (K=%d)", K);
-  // decode batches: the stream-K kernel (every CU streams an equal share of the weights, fixup kernel after)
-  if (!use_t8(M, N) && gemm_sk_applies(M, N, K, mode))
-    return launch_gemm_sk(A, lda, wt, N, K, C, ldc, M, mode, ws, ws_bytes, st);
-  if (use_t8(M, N)) {
-    const size_t need = gemm_t_workspace(M, N, K, mode), t8ws = gemm_t8_workspace(M, N, K);
+  // prefill, then decode batches with the stream-K kernel (every CU streams an equal share of the weights)
+  if (gemm_w_applies(M, N, K, mode)) {
+    const size_t need = gemm_t_workspace(M, N, K, mode);
     if (need > ws_bytes || (need && !ws))
       return fail(IFD_ERR_WORKSPACE, "gemm_t64 needs %zu bytes of workspace, got %zu", need, ws_bytes);
-    if (mode != kModeSwiglu) return launch_gemm_t8(A, lda, wt, N, K, C, ldc, M, mode, ws, t8ws, st);
-    // SwiGLU: the bf16 product into the workspace (after the tail partials), then silu_mul
-    uint16_t* gu = (uint16_t*)((char*)ws + align_up(t8ws, 256));
-    IFD_TRY(launch_gemm_t8(A, lda, wt, N, K, gu, N, M, 0, ws, t8ws, st));
-    return launch_silu_mul(gu, N, (uint16_t*)C, ldc, N / 2, M, st);
+    return launch_gemm_w(A, lda, wt, N, K, C, ldc, M, mode, ws, ws_bytes, st);
   }
+  if (gemm_sk_applies(M, N, K, mode))
+    return launch_gemm_sk(A, lda, wt, N, K, C, ldc, M, mode, ws, ws_bytes, st);
   const GtPlan pl = gemm_t_plan(M, N, K);
   const size_t need = epilogue_ws_bytes(pl.S, M, N, mode);
   if (need > ws_bytes || (need && !ws))

@@ -70,10 +70,11 @@ int launch_pack_t64(const uint32_t* wq, const uint16_t* s, const uint16_t* b, in
                     int E, void* out, hipStream_t st);
 size_t qmv_t_workspace(int M, int N, int K, int mode, int bits = 4);
 size_t gemm_t_workspace(int M, int N, int K, int mode);
-// 256-row-tile prefill GEMM on T64 weights (modes 0-2); gemm_t routes prefill shapes to it.
-size_t gemm_t8_workspace(int M, int N, int K);
-int launch_gemm_t8(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
-                   void* ws, size_t ws_bytes, hipStream_t st);
+// Prefill GEMM on T64 weights (gemm_w.hip): M > 128, modes 0-2 and SwiGLU.
+bool gemm_w_applies(int M, int N, int K, int mode);
+size_t gemm_w_workspace(int M, int N, int K);
+int launch_gemm_w(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
+                  void* ws, size_t ws_bytes, hipStream_t st);
 int launch_gemm_t(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
                   void* ws, size_t ws_bytes, hipStream_t st);
 // Stream-K GEMM for decode batches (gemm_sk.hip): every CU streams an equal share of the weights; the cut tiles are

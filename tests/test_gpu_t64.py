@@ -534,6 +534,53 @@ def test_gemm_t64_swiglu_prefill_tiles():
     assert np.array_equal(g.host(ops.gemm_t64_swiglu(A, T)), g.host(ops.silu_mul(ops.gemm_t64(A, T))))
 
 
+@pytest.mark.parametrize("M,N,K,mode,off", [
+    (129, 1024, 1024, 0, 0),    # one tile of 160 rows, 31 of them past M; every tile shared by several blocks
+    (160, 1040, 1024, 1, 0),    # whole 160-row tiles; the last band is half past N (16-byte stores stop there)
+    (161, 2048, 512, 2, 0),     # 192-row tiles; 4 groups per share
+    (225, 1028, 1024, 1, 0),    # N % 16 != 0: one value at a time
+    (256, 34816, 256, 0, 0),    # 136 tiles of 256 or more rows, no cut: half the CUs
+    (257, 16640, 1024, 1, 0),   # shares that cross a tile's end (two pieces per block)
+    (300, 17408, 1024, 0, 0),
+    (777, 13312, 512, 2, 0),    # whole tiles, then cut ones
+    (600, 768, 4096, 1, 1),     # a base and row stride that allow no 16-byte accesses
+    (1025, 16387, 256, 2, 0),   # odd N
+])
+def test_gemm_t64_prefill(M, N, K, mode, off):
+    """The prefill kernel (M > 128) against the qmm oracle on sampled rows: row-tile heights, tiles cut in shares that do
+    or do not end with a tile, partial bands, and every way its rows are stored. Repeated calls give the same bits."""
+    g, ops = _gu(), _ops()
+    from inferd_amd._lib import check, lib
+    codes, wq, s, b = gen.qlinear(N, K, seed=M + N + K)
+    T = ops.pack_t64(g.qlinear(wq, s, b))
+    A = gen.activations(M, K, seed=M + 3)
+    C0 = gen.activations(M, N + off, seed=M + 4)
+    ws = ops.workspace(lib().ifd_gemm_t64_workspace(M, N, K), "cuda")
+    Ad, outs = g.dev(A), []
+    for _ in range(2):
+        wide = torch.zeros((M, N + off), dtype=torch.float32, device="cuda") if mode == 2 else g.dev(C0)
+        check(lib().ifd_gemm_t64(Ad.data_ptr(), K, T.wt.data_ptr(), N, K, wide[:, off:].data_ptr(), N + off, M, mode,
+                                 ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+        outs.append(g.host(wide))
+    assert np.array_equal(outs[0], outs[1])
+    if mode != 2:
+        assert np.array_equal(outs[0][:, :off], C0[:, :off]), "stores outside the columns"
+    rows = np.unique(np.r_[np.linspace(0, M - 1, 9).astype(int), M - 2])
+    Y = orc.qmm(np.ascontiguousarray(A[rows]), wq, s, b)
+    ref = Y + gen.bf16_to_f32(C0[rows][:, off:]) if mode == 1 else Y
+    gen.check_out(outs[0][rows][:, off:], ref, 1e-2, (M, N, K, mode, off), fp32=mode == 2)
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 17408, 1024), (777, 9216, 512), (1025, 16384, 256)])
+def test_gemm_t64_prefill_swiglu_bits(M, N, K):
+    """The fused gate/up entry at M > 128, also where its tiles are cut: the bits of gemm_t64 + silu_mul."""
+    g, ops = _gu(), _ops()
+    codes, wq, s, b = gen.qlinear(N, K, seed=M + K)
+    A = g.dev(gen.activations(M, K, seed=M + 1))
+    T = ops.pack_t64(g.qlinear(wq, s, b))
+    assert np.array_equal(g.host(ops.gemm_t64_swiglu(A, T)), g.host(ops.silu_mul(ops.gemm_t64(A, T))))
+
+
 # ---- the dense decode MLP block -----------------------------------------------------------------------------------
 @pytest.mark.parametrize("M", [1, 8, 32, 128])
 def test_mlp_decode_matches_its_sequence_at_config1(M):
