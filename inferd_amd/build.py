@@ -17,7 +17,7 @@ MOE_BENCH_SRC = os.path.join(HERE, "csrc", "encode_moe_bench.cpp")
 MOE_BENCH = os.path.join(HERE, "encode_moe_bench")
 OBJ = os.path.join(HERE, "_build")
 
-SOURCES = ["qmv.hip", "qmm.hip", "w4a8.hip", "moe.hip", "t64.hip", "gemm_t64.hip", "gemm_sk.hip", "gemm_w.hip",
+SOURCES = ["qmv.hip", "qmm.hip", "w4a8.hip", "moe.hip", "t64.hip", "gemm_t64.hip", "gemm_sk.hip", "gemm_w.hip", "gemm_n.hip",
            "w4a8_t64.hip", "w8a8_t64.hip", "fused.hip", "moe_dec.hip", "moe_t64.hip", "capi.hip", "workspace.hip",
            "probe.hip", "noalloc.hip"]
 

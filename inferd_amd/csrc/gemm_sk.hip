@@ -1,8 +1,7 @@
-// Stream-K GEMM on T64 weights for decode batches (16 < M, below the 256-row prefill tiles): C (mode) = A . W^T with
-// every weight dequantized to bf16(s q + b) (MLX qmm rounding, third_party/mlx/.../quantized.h:528-535) and fp32
-// accumulation. Serves the reference's affine_qmm_t_nax (quantized_nax.h:938-1076) with its split-K variant
-// (engine/kernels/qmm_splitk.metal:14-107) and, in the SwiGLU mode, the gemm -> silu_mul pair of the MLP
-// (engine/src/qwen35.h:1693-1700).
+// Stream-K GEMM on T64x8 (8-bit) weights past the decode GEMV's rows: C (mode) = A . W^T with every weight dequantized
+// to bf16(s q + b) (MLX 8-bit qmm rounding, third_party/mlx/.../quantized.h:528-535) and fp32 accumulation. Serves the
+// reference's affine_qmm_t_nax (quantized_nax.h:938-1076) with its split-K variant
+// (engine/kernels/qmm_splitk.metal:14-107) at BITS = 8. (The BITS = 4 form served T64 decode batches; gemm_n.hip does.)
 //
 // Work is the set of units (tile, 64-group); a tile is BM = 32 MT rows x 8 bands (256 columns). Block b (of nblk,
 // one or two per CU) takes units [b U / nblk, (b + 1) U / nblk) (stream-K): every CU streams the same weight bytes
@@ -27,8 +26,7 @@
 // SwiGLU mode: tile t holds gate bands 4t..4t+3 (waves 0, 1) and the matching up bands (waves 2, 3); the staged tile
 // (or the fixup) gives h = silu(bf16(gate)) * bf16(up) (reference silu_mul, core.metal:777-787).
 //
-// The same kernel serves T64x8 (8-bit) weights with BITS = 8: a band's codes are two 1 KB halves per group (two DMAs
-// instead of one), dequantized from the stored q - 128 bytes to bf16(s q + b), MLX's 8-bit qmm rounding.
+// A band's codes are two 1 KB halves per group, dequantized from the stored q - 128 bytes to bf16(s q + b).
 #include <algorithm>
 #include <type_traits>
 
@@ -602,13 +600,6 @@ static int launch_sk_bits(const uint16_t* A, int lda, const void* wt, int N, int
   if (pl.MT == 1) return launch_sk_cfg<1, BITS>(a, fixup, st);
   if (pl.MT == 2) return launch_sk_cfg<2, BITS>(a, fixup, st);
   return launch_sk_cfg<4, BITS>(a, fixup, st);
-}
-
-int launch_gemm_sk(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
-                   void* ws, size_t ws_bytes, hipStream_t st) {
-  if (M == 0) return IFD_OK;
-  if (!gemm_sk_applies(M, N, K, mode)) return fail(IFD_ERR_UNSUPPORTED, "gemm_sk: shape M=%d N=%d K=%d", M, N, K);
-  return launch_sk_bits<4>(A, lda, wt, N, K, C, ldc, M, mode, ws, ws_bytes, st);
 }
 
 int launch_gemm_sk8(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,

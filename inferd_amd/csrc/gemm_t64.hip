@@ -312,7 +312,20 @@ static GtPlan gemm_t_plan(int M, int N, int K, int Mrows = 0) {
   return pl;
 }
 
+// Past 16 rows the decode GEMV's arithmetic goes on up to 64 rows where there are few column tiles (the stream-K rule's
+// complement), as it always has; elsewhere the weights are rounded to bf16.
+static bool gemm_n_affine(int M, int N, int K, int mode) { return M <= 64 && !gemm_sk_applies(M, N, K, mode); }
+
+// Past 16 rows a gate/up pair whose halves are no whole bands of the kernels below runs as the plain GEMM into the
+// workspace, then silu_mul.
+static bool swiglu_by_product(int M, int N, int K, int mode) {
+  return mode == kModeSwiglu && !gemm_w_applies(M, N, K, mode) && !gemm_n_applies(M, N, K, mode) &&
+         (gemm_w_applies(M, N, K, 0) || gemm_n_applies(M, N, K, 0));
+}
+
 size_t gemm_t_workspace(int M, int N, int K, int mode) {
+  if (swiglu_by_product(M, N, K, mode))
+    return align_up(gemm_t_workspace(M, N, K, 0), 256) + (size_t)M * N * sizeof(uint16_t);
   // The size of a prefill shape decides which requests the static scratch of ifd_gemm_t64_noalloc serves, so it is never
   // less than a split of 256-row tiles (from a round of them) or the stream-K kernel (below) would need.
   if (gemm_w_applies(M, N, K, mode)) {
@@ -322,8 +335,9 @@ size_t gemm_t_workspace(int M, int N, int K, int mode) {
     else if (tail && tail <= 128) least = (size_t)std::min({256 / tail, 8L, K / kGroup / 4L}) * tail * 256 * 256 * 4;
     return std::max(gemm_w_workspace(M, N, K), least);
   }
-  if (gemm_sk_applies(M, N, K, mode)) return gemm_sk_workspace(M, N, K, mode);
-  return epilogue_ws_bytes(gemm_t_plan(M, N, K).S, M, N, mode);
+  const size_t least =
+      gemm_sk_applies(M, N, K, mode) ? gemm_sk_workspace(M, N, K, mode) : epilogue_ws_bytes(gemm_t_plan(M, N, K).S, M, N, mode);
+  return gemm_n_applies(M, N, K, mode) ? std::max(gemm_n_workspace(M, N, K, gemm_n_affine(M, N, K, mode)), least) : least;
 }
 
 template <int MT, int NB, bool DEQ, bool A8 = false>
@@ -371,15 +385,19 @@ int launch_gemm_t(const uint16_t* A, int lda, const void* wt, int N, int K, void
                   void* ws, size_t ws_bytes, hipStream_t st) {
   if (M == 0) return IFD_OK;
   if (K % 128) return fail(IFD_ERR_ARG, "T64 GEMM needs K %% 128 == 0 (K=%d)", K);
-  // prefill, then decode batches with the stream-K kernel (every CU streams an equal share of the weights)
-  if (gemm_w_applies(M, N, K, mode)) {
+  const bool by_product = swiglu_by_product(M, N, K, mode);
+  const bool w = gemm_w_applies(M, N, K, mode), n = gemm_n_applies(M, N, K, mode);
+  if (by_product || w || n) {
     const size_t need = gemm_t_workspace(M, N, K, mode);
     if (need > ws_bytes || (need && !ws))
       return fail(IFD_ERR_WORKSPACE, "gemm_t64 needs %zu bytes of workspace, got %zu", need, ws_bytes);
-    return launch_gemm_w(A, lda, wt, N, K, C, ldc, M, mode, ws, ws_bytes, st);
+    if (w) return launch_gemm_w(A, lda, wt, N, K, C, ldc, M, mode, ws, ws_bytes, st);
+    if (n) return launch_gemm_n(A, lda, wt, N, K, C, ldc, M, mode, gemm_n_affine(M, N, K, mode), ws, ws_bytes, st);
+    const size_t plain = gemm_t_workspace(M, N, K, 0);
+    uint16_t* gu = (uint16_t*)((char*)ws + align_up(plain, 256));
+    IFD_TRY(launch_gemm_t(A, lda, wt, N, K, gu, N, M, 0, ws, plain, st));
+    return launch_silu_mul(gu, N, (uint16_t*)C, ldc, N / 2, M, st);
   }
-  if (gemm_sk_applies(M, N, K, mode))
-    return launch_gemm_sk(A, lda, wt, N, K, C, ldc, M, mode, ws, ws_bytes, st);
   const GtPlan pl = gemm_t_plan(M, N, K);
   const size_t need = epilogue_ws_bytes(pl.S, M, N, mode);
   if (need > ws_bytes || (need && !ws))

@@ -20,7 +20,7 @@
 //   tile's stores overlap the next tile's first loads. Where the last round's tiles would leave CUs idle their groups
 //   are shared out evenly among S blocks per tile or among all CUs: a block then sums its one or two pieces first (fp32,
 //   to slots), and k_gemm_w_fixup adds a tile's pieces in K order. w_plan picks MT and the split by estimated time; over
-//   60 drawn shapes of 129 to 4096 rows no forced choice beat it by more than 4%.
+//   twelve swept shapes no forced choice beat it by more than 4%.
 // - Weights are the MFMA's A operand, so a lane holds four neighbouring columns of one row: with v_permlane32_swap
 //   bf16 rows leave as 16-byte stores straight from the registers.
 // Columns: where N % 256 == 0 a tile is bands 4 t .. + 3 of the left half of the columns and the same bands of the
@@ -39,6 +39,7 @@
 #include "dma.h"
 #include "host.h"
 #include "kernels.h"
+#include "share.h"
 #include "t64.h"
 #include "t64_dev.h"
 
@@ -66,16 +67,6 @@ struct GemmWArgs {
   int full;           // tiles 0 .. full - 1 are summed whole, block b taking b, b + gridDim.x, ..
   int rem, nsk;       // the rem other tiles' groups are shared evenly among blocks 0 .. nsk - 1 (rem < nsk)
 };
-
-// The shares of the cut tiles' rem G groups: block b's starts at group w_share(b), group u is in block w_share_of(u)'s.
-// A share is shorter than a tile, so it is part of at most two. The pieces in order are numbered by block where every
-// tile is cut at the same groups (nsk a multiple of rem), else by block + tile.
-__host__ __device__ inline int w_share(int b, int rem, int nsk, int G) { return (int)((long)b * rem * G / nsk); }
-__host__ __device__ inline int w_share_of(int u, int rem, int nsk, int G) {
-  return (int)(((long)u * nsk + nsk - 1) / ((long)rem * G));
-}
-__host__ __device__ inline int w_piece(int b, int tile, int rem, int nsk) { return nsk % rem ? b + tile : b; }
-__host__ __device__ inline int w_pieces(int rem, int nsk) { return rem == 0 ? 0 : nsk % rem ? nsk + rem - 1 : nsk; }
 
 // tile order: bands of kWBand M tiles, M fastest, so that neighbouring blocks (one XCD) share weight tiles in L2
 __host__ __device__ inline void w_tile(int L, int tiles_m, int tiles_n, int& tm, int& tn) {
@@ -214,7 +205,7 @@ __global__ __launch_bounds__(256, 1) void k_gemm_w(GemmWArgs p) {
   // the block's segments: its share of the cut tiles (one or two pieces), then its whole tiles
   int u0 = 0, u1 = 0, hp = 0;
   if (b < p.nsk) {
-    u0 = w_share(b, p.rem, p.nsk, G), u1 = w_share(b + 1, p.rem, p.nsk, G);
+    u0 = share_start(b, p.rem, p.nsk, G), u1 = share_start(b + 1, p.rem, p.nsk, G);
     hp = (u1 - 1) / G > u0 / G ? 2 : 1;
   }
   const int nseg = hp + (b < p.full ? (p.full - 1 - b) / nblk + 1 : 0);
@@ -385,7 +376,7 @@ __global__ __launch_bounds__(256, 1) void k_gemm_w(GemmWArgs p) {
     // the segment's sums: lane (j, h) holds row 32 a + j, columns 8 q + 4 h + e of its two bands (kWScalar: the converse)
     if (s < hp) {
       float4* const slot =
-          (float4*)p.part + (size_t)w_piece(b, t - p.full, p.rem, p.nsk) * 8 * MT * 4 * 64 + lane;
+          (float4*)p.part + (size_t)share_piece(b, t - p.full, p.rem, p.nsk) * 8 * MT * 4 * 64 + lane;
 #pragma unroll
       for (int nb = 0; nb < 2; nb++)
 #pragma unroll
@@ -437,9 +428,9 @@ __global__ __launch_bounds__(256) void k_gemm_w_fixup(GemmWArgs p) {
   w_tile(p.full + blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
   if (tm * 32 * MT + 32 * a >= p.M) return;
   const int tile = blockIdx.x, G = p.K / kGroup;
-  const int b0 = w_share_of(tile * G, p.rem, p.nsk, G), b1 = w_share_of(tile * G + G - 1, p.rem, p.nsk, G);
+  const int b0 = share_of(tile * G, p.rem, p.nsk, G), b1 = share_of(tile * G + G - 1, p.rem, p.nsk, G);
   const float4* const slot =
-      (const float4*)p.part + (size_t)w_piece(b0, tile, p.rem, p.nsk) * 8 * MT * 4 * 64 + lane;
+      (const float4*)p.part + (size_t)share_piece(b0, tile, p.rem, p.nsk) * 8 * MT * 4 * 64 + lane;
   f32x16 x[2] = {zero16(), zero16()};
   WOld old;
   if (p.mode == 1) w_load_old<ST>(p, tm * 32 * MT + 32 * a + j, tn, wave, j, h, old);
@@ -486,7 +477,7 @@ static WPlan w_plan_mt(int MT, int M, int N, int K, size_t part_bytes) {
   // the last round's tiles shared by S blocks each, or (S = 0) by all CUs
   for (int S = 0; rem && S <= std::min(cu / rem, 16); S++) {
     const int nsk = S ? rem * S : cu;
-    const size_t bytes = (size_t)w_pieces(rem, nsk) * w_slot_bytes(MT);
+    const size_t bytes = (size_t)share_pieces(rem, nsk) * w_slot_bytes(MT);
     const double share = (double)rem * G / nsk;
     if (S == 1 || share < 4 || bytes > part_bytes) continue;
     const double ns = whole + std::ceil(share) * step + kWSegment * (nsk % rem ? 1.5 : 1) + kWFixup +
@@ -514,7 +505,7 @@ bool gemm_w_applies(int M, int N, int K, int mode) {
 
 size_t gemm_w_workspace(int M, int N, int K) {
   const WPlan pl = w_plan(M, N, K, kWPartMax);
-  return (size_t)w_pieces(pl.rem, pl.nsk) * w_slot_bytes(pl.MT);
+  return (size_t)share_pieces(pl.rem, pl.nsk) * w_slot_bytes(pl.MT);
 }
 
 template <int MT, int ST>
@@ -548,7 +539,7 @@ int launch_gemm_w(const uint16_t* A, int lda, const void* wt, int N, int K, void
   if (M == 0) return IFD_OK;
   if ((size_t)M * lda * 2 >= ((size_t)1 << 31)) return fail(IFD_ERR_UNSUPPORTED, "gemm_w: operands past 2 GiB");
   const WPlan pl = w_plan(M, N, K, kWPartMax);
-  const size_t need = (size_t)w_pieces(pl.rem, pl.nsk) * w_slot_bytes(pl.MT);
+  const size_t need = (size_t)share_pieces(pl.rem, pl.nsk) * w_slot_bytes(pl.MT);
   if (need > ws_bytes || (need && !ws))
     return fail(IFD_ERR_WORKSPACE, "gemm_w needs %zu bytes of workspace, got %zu", need, ws_bytes);
   GemmWArgs a{A, lda, (const uint8_t*)wt, (uint32_t)t64_bytes(N, K), N, K, C, ldc, M, mode, (float*)ws, pl.tiles_m,

@@ -75,14 +75,18 @@ bool gemm_w_applies(int M, int N, int K, int mode);
 size_t gemm_w_workspace(int M, int N, int K);
 int launch_gemm_w(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
                   void* ws, size_t ws_bytes, hipStream_t st);
+// GEMM on T64 weights for 16 < M <= 128 (gemm_n.hip), modes 0-2 and SwiGLU; affine: the decode GEMV's arithmetic
+// (up to 64 rows), else bf16-dequantized weights.
+bool gemm_n_applies(int M, int N, int K, int mode);
+size_t gemm_n_workspace(int M, int N, int K, bool affine);
+int launch_gemm_n(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
+                  bool affine, void* ws, size_t ws_bytes, hipStream_t st);
 int launch_gemm_t(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
                   void* ws, size_t ws_bytes, hipStream_t st);
-// Stream-K GEMM for decode batches (gemm_sk.hip): every CU streams an equal share of the weights; the cut tiles are
-// summed by a fixup kernel.
+// The stream-K plan (gemm_sk.hip) of a 4-bit shape: whether it has tiles for a third of the CUs (or one 128-row tile),
+// and its workspace, which decode batches still report (their callers' buffers have that size).
 bool gemm_sk_applies(int M, int N, int K, int mode);
 size_t gemm_sk_workspace(int M, int N, int K, int mode);
-int launch_gemm_sk(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
-                   void* ws, size_t ws_bytes, hipStream_t st);
 // The fixup of a 128-row-tile stream-K split (gemm_sk.hip): sums the pieces of the cut tiles among the stream-K
 // tiles tile0 .. tile0 + ntiles - 1, scales row m by rs[m rs_stride] (rs null: no scale) and stores them.
 int launch_sk_fixup_rows(const float* part, int tiles_m, int tiles_n, int tile0, int ntiles, int G, int nblk, void* C,
@@ -95,7 +99,7 @@ int launch_w4a8_t(const int8_t* U, const float* XS, const void* wt, int N, int K
 // is qmv_t_workspace(M, N, K, mode, 8).
 int launch_qmv_t8(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
                   unsigned* cnt, void* ws, size_t ws_bytes, hipStream_t st);
-// The same stream-K GEMM on T64x8 weights (8-bit codes, dequantized to bf16(s q + b)); any M >= 1.
+// Stream-K GEMM (gemm_sk.hip) on T64x8 weights (8-bit codes, dequantized to bf16(s q + b)); any M >= 1.
 size_t gemm_sk8_workspace(int M, int N, int K);
 int launch_gemm_sk8(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
                     void* ws, size_t ws_bytes, hipStream_t st);

@@ -581,6 +581,46 @@ def test_gemm_t64_prefill_swiglu_bits(M, N, K):
     assert np.array_equal(g.host(ops.gemm_t64_swiglu(A, T)), g.host(ops.silu_mul(ops.gemm_t64(A, T))))
 
 
+@pytest.mark.parametrize("M,N,K,mode", [
+    (17, 33, 256, 0),        # affine; one 128-column tile, two live bands (the second one column wide); one round of K
+    (32, 1000, 2048, 1),     # shared tiles, N off the bands: neighbouring bands per tile
+    (32, 23040, 768, 2),     # dequantized at 32 rows; 3 rounds
+    (33, 1024, 768, 2),      # affine past 32 rows
+    (64, 5120, 1280, 1),     # 5 rounds over 6 shares a tile
+    (64, 23040, 512, 0),     # dequantized at 64 rows; no cut
+    (65, 640, 4352, 2),      # 96-row tiles, 17 rounds
+    (96, 33024, 256, 1),     # 258 tiles: two of them shared, one round of K each
+    (97, 4096, 1024, 0),     # 128-row tiles
+    (128, 34816, 512, 2),    # whole tiles and shared ones
+    (128, 131, 1024, 1),     # odd N
+])
+def test_gemm_t64_decode_batches(M, N, K, mode):
+    """The decode-batch kernel (16 < M <= 128) against the oracle: row tiles, tiles summed whole, shared out and both,
+    register-set turns with every remainder, partial bands, every store mode. Repeated calls give the same bits."""
+    g, ops = _gu(), _ops()
+    codes, wq, s, b = gen.qlinear(N, K, seed=M + N + K)
+    T = ops.pack_t64(g.qlinear(wq, s, b))
+    A = gen.activations(M, K, seed=M + 3)
+    C0 = gen.activations(M, N, seed=M + 4)
+    outs = [g.host(ops.gemm_t64(g.dev(A), T, g.dev(C0) if mode == 1 else None, mode=mode)) for _ in range(2)]
+    assert np.array_equal(outs[0], outs[1])
+    rows = np.unique(np.r_[np.linspace(0, M - 1, 9).astype(int), M - 2])
+    Y = _t64_arith(M, N, K)(np.ascontiguousarray(A[rows]), wq, s, b)
+    ref = Y + gen.bf16_to_f32(C0[rows]) if mode == 1 else Y
+    gen.check_out(outs[0][rows], ref, 1e-2, (M, N, K, mode), fp32=mode == 2)
+
+
+@pytest.mark.parametrize("M,N,K", [(20, 1056, 512), (100, 34816, 256), (100, 1056, 512), (200, 1056, 512)])
+def test_gemm_t64_swiglu_past_16_rows(M, N, K):
+    """Gate/up pairs with whole bands per half and without (product, then silu_mul): the SwiGLU of the plain product,
+    bit for bit where both cut K alike."""
+    g, ops = _gu(), _ops()
+    codes, wq, s, b = gen.qlinear(N, K, seed=M + N)
+    A = g.dev(gen.activations(M, K, seed=M + 1))
+    T = ops.pack_t64(g.qlinear(wq, s, b))
+    assert np.array_equal(g.host(ops.gemm_t64_swiglu(A, T)), g.host(ops.silu_mul(ops.gemm_t64(A, T))))
+
+
 # ---- the dense decode MLP block -----------------------------------------------------------------------------------
 @pytest.mark.parametrize("M", [1, 8, 32, 128])
 def test_mlp_decode_matches_its_sequence_at_config1(M):
