@@ -17,12 +17,17 @@
 //   slabs per K-group.
 // FORM 0: weights dequantized to bf16(s q + b) (MLX qmm rounding, quantized.h:528-535), in place, one sub-step behind
 // the MFMAs. FORM 1: the decode GEMV's arithmetic (core.metal:85-171): 128 + q as exact bf16, and per 64-group the fp32
-// epilogue adds s P + (b - 128 s) X, X from an MFMA against ones.
+// epilogue adds s P + (b - 128 s) X, X from an MFMA against ones. FORM 2: the reference's W4A8 with per-(row, 64-group)
+// int8 activations (w4a8.metal:24-98): A holds the codes xq as exact bf16 integers, so P = sum (128 + q) xq and
+// X = sum xq are exact (integers below 2^24), and the epilogue adds sx (s P + (b - 128 s) X) with the row's scale for
+// that group; more than 64 rows are blocks of 64, neighbours in the tile order.
 // What bounds it: at 128 rows the power-limited MFMA rate (1.65 us per round of 4 units, 1.3 PFLOP/s) and about 12 us of
 // first loads, sums and stores; below, the weight stream (0.9 us per round at 32 rows for 0.8 at 6 TB/s). Measured,
 // whole call, same box, before (stream-K or K-split tiles) -> after: 32768 x 5120 at M = 128 / 64 / 32 58.2 / 40.7 /
 // 33.1 -> 45.1 / 32.1 / 25.4 us; gate and up with SwiGLU, 34816 x 5120 (16 shared tiles), 62.5 / 43.0 / 36.0 -> 59.8 /
 // 41.6 / 32.4; 5120 x 17408 42.9 / 32.0 / 25.8 -> 37.4 / 27.2 / 20.3; 34 drawn shapes 1.05 to 1.86 times, 1.36 in the mean.
+// FORM 2 (with its prep), before the K-split tiles: 34816 x 5120 at M = 24 / 64 / 128 / 255 53.8 / 86.3 / 123.6 / 215.8 ->
+// 38.7 / 51.0 / 84.9 / 154.3 us; 5120 x 17408 at M = 24 27.8 -> 26.8.
 // Deeper register sets (NS 5 to 7) measured slower at 32 and 64 rows.
 // Activation slabs: [32 MT][64 bf16], 16-byte columns XOR-swizzled by row pair, filled by direct global -> LDS DMA, each
 // issued by a whole wave under wave-uniform control flow (the LDS base goes to M0).
@@ -41,7 +46,10 @@
 namespace ifd {
 
 __host__ __device__ constexpr int n_ra(int MT) { return MT == 4 ? 2 : MT == 3 ? 3 : 4; }
-__host__ __device__ constexpr int n_lds(int MT, int NKQ) { return NKQ * n_ra(MT) * MT * 4096; }
+__host__ __device__ constexpr int n_ring(int MT, int NKQ) { return NKQ * n_ra(MT) * MT * 4096; }
+__host__ __device__ constexpr int n_lds(int MT, int NKQ, int FORM) {
+  return n_ring(MT, NKQ) + (FORM == 2 ? NKQ * (n_ra(MT) + 1) * 256 : 0);
+}
 __host__ __device__ constexpr size_t n_slot_bytes(int MT) { return (size_t)4 * MT * 16 * 64 * sizeof(float); }
 
 struct GemmNArgs {
@@ -52,6 +60,9 @@ struct GemmNArgs {
   int N, K;
   void* C;
   int ldc, M, mode;
+  const float* sxT;   // FORM 2: the activation scales transposed, [G][Mp], Mp >= 64 tiles_m + 64
+  int Mp;
+  int tiles_m;        // row blocks of 32 MT (row block fastest in the tile order)
   float* part;        // piece slots [][2 waves][2 bands][MT * 4][64] float4
   int half;           // bands per half of the columns (N % 128 == 0), or 0: a tile is 4 neighbouring bands
   int full;           // tiles 0 .. full - 1 are summed whole, block b taking b, b + gridDim.x, ..
@@ -105,13 +116,20 @@ template <int MT, int NKQ, int FORM, int NS, int MODE>
 __global__ __launch_bounds__(128 * NKQ, 1) void k_gemm_n(GemmNArgs p) {
   extern __shared__ __align__(16) uint8_t lds[];
   constexpr int RA = n_ra(MT), AB = MT * 4096;
-  static_assert((RA - 1) * 4 + (RA - 2) * 2 * MT <= 63 && n_lds(MT, NKQ) <= 160 * 1024, "vmcnt range, LDS");
+  constexpr int SX = FORM == 2 ? 1 : 0;
+  static_assert((RA - 1) * 4 + (RA - 2) * (2 * MT + SX) <= 63 && n_lds(MT, NKQ, FORM) <= 160 * 1024, "vmcnt range, LDS");
+  static_assert(FORM != 2 || MT <= 2, "one scale DMA covers 64 rows");
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kq = wv >> 1, w = wv & 1;
   const int lane = threadIdx.x & 63, j = lane & 31, h = lane >> 5;
   const int b = xcd_remap(blockIdx.x, gridDim.x), nblk = gridDim.x;
   const int nbands = t64_bands(p.N), R = p.K / kGroup / NKQ;  // rounds per tile
   const uint32_t gstride = (uint32_t)nbands * kT64Tile;
   uint8_t* const ring = lds + kq * RA * AB;
+  // FORM 2: the units' row scales, RA + 1 slots of 64 floats: a slot is refilled a unit later than its slab, when both
+  // waves are past the epilogue that read it
+  uint8_t* const sxring = lds + n_ring(MT, NKQ) + kq * (RA + 1) * 256;
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)p.sxT, 0, FORM == 2 ? (int)((uint32_t)(p.K / kGroup) * p.Mp * 4u) : 0, 0x00020000);
   const __amdgpu_buffer_rsrc_t ra =
       __builtin_amdgcn_make_buffer_rsrc((void*)p.A, 0, (int)((uint32_t)p.M * p.lda * 2u), 0x00020000);
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)p.wt, 0, (int)p.w_bytes, 0x00020000);
@@ -164,7 +182,7 @@ __global__ __launch_bounds__(128 * NKQ, 1) void k_gemm_n(GemmNArgs p) {
     segment(sg, t, r0, w_left);
     w_so = (uint32_t)(r0 * NKQ + kq) * gstride;
 #pragma unroll
-    for (int nb = 0; nb < 2; nb++) vw[nb] = (uint32_t)min(n_band(p, t, w, nb), nbands - 1) * kT64Tile;
+    for (int nb = 0; nb < 2; nb++) vw[nb] = (uint32_t)min(n_band(p, t / p.tiles_m, w, nb), nbands - 1) * kT64Tile;
     static_for<0, FORM == 0 ? NS : NS - 1>([&](auto SC) __attribute__((always_inline)) { load_w(SC); });
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -175,12 +193,22 @@ __global__ __launch_bounds__(128 * NKQ, 1) void k_gemm_n(GemmNArgs p) {
   for (int sg = 0; sg < nseg; sg++) {
     int t, r0, nr;
     segment(sg, t, r0, nr);
+    const int tm = t % p.tiles_m, tn = t / p.tiles_m;
+    const uint32_t m_off = (uint32_t)tm * 32u * MT * p.lda * 2u;
     uint32_t a_so = (uint32_t)(r0 * NKQ + kq) * 2u * kGroup;
     int a_left = nr;
-    auto adv_a = [&]() __attribute__((always_inline)) { a_so += --a_left > 0 ? 2u * kGroup * NKQ : 0u; };
+    uint32_t x_so = ((uint32_t)(r0 * NKQ + kq) * p.Mp + (uint32_t)tm * 32u * MT) * 4u;
+    auto adv_a = [&]() __attribute__((always_inline)) {
+      const bool on = --a_left > 0;
+      a_so += on ? 2u * kGroup * NKQ : 0u;
+      if constexpr (FORM == 2) x_so += on ? (uint32_t)p.Mp * 4u * NKQ : 0u;
+    };
+    auto issue_x = [&](int slot) __attribute__((always_inline)) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void_t*)(sxring + slot), 4, 4 * lane, (int)x_so, 0, 0);
+    };
     auto issue_a = [&](uint8_t* st, int d) __attribute__((always_inline)) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void_t*)(st + (2 * MT * w + d) * 1024), 16,
-                                               (int)(va[d & 1] + (uint32_t)(d & ~1) * 16u * p.lda), (int)a_so, 0, 0);
+                                               (int)(va[d & 1] + m_off + (uint32_t)(d & ~1) * 16u * p.lda), (int)a_so, 0, 0);
     };
 
     f32x16 acc[2][MT], P[2][MT], X[MT];
@@ -197,9 +225,12 @@ __global__ __launch_bounds__(128 * NKQ, 1) void k_gemm_n(GemmNArgs p) {
     for (int s = 0; s < RA; s++) {
 #pragma unroll
       for (int d = 0; d < (s + 1 < RA ? 2 * MT : MT); d++) issue_a(ring + s * AB, d);
-      if (s + 1 < RA) adv_a();
+      if (s + 1 < RA) {
+        if constexpr (FORM == 2) issue_x(s * 256);
+        adv_a();
+      }
     }
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((RA - 2) * 2 * MT + MT) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((RA - 2) * (2 * MT + SX) + MT) : "memory");
 #pragma unroll
     for (int a = 0; a < MT; a++) af[a] = *(const u32x4*)(ring + asw + a * 4096);
     auto scales = [&](uint32_t x, int nb) __attribute__((always_inline)) {
@@ -220,10 +251,10 @@ __global__ __launch_bounds__(128 * NKQ, 1) void k_gemm_n(GemmNArgs p) {
     // One unit i (SC = i mod NS); offsets of its slab, the one before and after. Sub-step k issues, after barriers as in
     // the comment of each: the second half of A(i + RA - 1) (k = 0), W(i + NS) or, FORM 1, W(i + NS - 1) into the
     // registers of W(i) or W(i - 1) (k = 1), the first half of A(i + RA) (k = 3, into the slab whose last fragments were read at k = 2).
-    int sl = 0, slp = (RA - 1) * AB, sln = AB;
+    int sl = 0, slp = (RA - 1) * AB, sln = AB, xr = 0, xw = (RA - 1) * 256;
     auto unit = [&](auto SC) __attribute__((always_inline)) {
       constexpr int S = decltype(SC)::value, S1 = (S + 1) % NS, SL = (S + NS - 1) % NS;
-      if constexpr (FORM == 1)
+      if constexpr (FORM != 0)
 #pragma unroll
         for (int nb = 0; nb < 2; nb++) scales(csb[S][nb], nb);
 #pragma unroll
@@ -234,10 +265,10 @@ __global__ __launch_bounds__(128 * NKQ, 1) void k_gemm_n(GemmNArgs p) {
         if (k == 1) load_w(std::integral_constant<int, FORM == 0 ? S : SL>{});
         // A(i + 1) has landed: younger are A(i + 2 .. i + RA - 1) and the weights of RA - 1 units
         if (k == 3)
-          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((RA - 1) * 4 + (RA - 2) * 2 * MT) : "memory");
+          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((RA - 1) * 4 + (RA - 2) * (2 * MT + SX)) : "memory");
         const uint8_t* const src = ring + ((asw ^ (16u * ((k + 1) & 3))) + (k == 3 ? sln : sl));
         const int kw = (k + 3) & 3;
-        if constexpr (FORM == 1)
+        if constexpr (FORM != 0)
 #pragma unroll
           for (int nb = 0; nb < 2; nb++) bf[nb][k] = t64_off128(cw[S][nb][k]);
 #pragma unroll
@@ -270,7 +301,13 @@ __global__ __launch_bounds__(128 * NKQ, 1) void k_gemm_n(GemmNArgs p) {
           }
           __builtin_amdgcn_sched_barrier(0);
         }
-        if (k == 0) adv_a();
+        if (k == 0) {
+          if constexpr (FORM == 2) {
+            issue_x(xw);
+            xw = xw == RA * 256 ? 0 : xw + 256;
+          }
+          adv_a();
+        }
       }
       if constexpr (FORM == 1)
 #pragma unroll
@@ -280,6 +317,22 @@ __global__ __launch_bounds__(128 * NKQ, 1) void k_gemm_n(GemmNArgs p) {
 #pragma unroll
             for (int e = 0; e < 16; e++)
               acc[nb][a][e] = __builtin_fmaf(sa[nb], P[nb][a][e], __builtin_fmaf(bi[nb], X[a][e], acc[nb][a][e]));
+      if constexpr (FORM == 2) {
+#pragma unroll
+        for (int a = 0; a < MT; a++)
+#pragma unroll
+          for (int c = 0; c < 4; c++) {
+            const float4 x = *(const float4*)(sxring + xr + (32 * a + 8 * c + 4 * h) * 4);
+            const float sx[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+            for (int nb = 0; nb < 2; nb++)
+#pragma unroll
+              for (int e = 0; e < 4; e++)
+                acc[nb][a][4 * c + e] = __builtin_fmaf(
+                    sx[e], __builtin_fmaf(sa[nb], P[nb][a][4 * c + e], bi[nb] * X[a][4 * c + e]), acc[nb][a][4 * c + e]);
+          }
+        xr = xr == RA * 256 ? 0 : xr + 256;
+      }
       slp = sl, sl = sln;
       sln = sln + AB == RA * AB ? 0 : sln + AB;
     };
@@ -294,7 +347,7 @@ __global__ __launch_bounds__(128 * NKQ, 1) void k_gemm_n(GemmNArgs p) {
 
     // ---- the K-groups' sums meet in LDS, PQ quads of rows (quad c: rows 8 c + 4 h .. + 3) at a time:
     // [K-group][wave][band][quad][lane] float4. K-group kq adds them, in K-group order, for quads kq, kq + NKQ, ..
-    constexpr int Q = 4 * MT, PQ = NKQ * Q * 4096 <= n_lds(MT, NKQ) ? Q : Q / 2;
+    constexpr int Q = 4 * MT, PQ = NKQ * Q * 4096 <= n_ring(MT, NKQ) ? Q : Q / 2;
     float4* const red = (float4*)lds;
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (sg + 1 < nseg) open_w(sg + 1);
@@ -329,7 +382,7 @@ __global__ __launch_bounds__(128 * NKQ, 1) void k_gemm_n(GemmNArgs p) {
           for (int nb = 0; nb < 2; nb++)
             slot[((w * 2 + nb) * Q + c0 + c) * 64] = make_float4(v[nb][0], v[nb][1], v[nb][2], v[nb][3]);
         } else {
-          n_emit<MODE>(p, t, w, 8 * (c0 + c) + 4 * h, j, v[0], v[1]);
+          n_emit<MODE>(p, tn, w, 32 * MT * tm + 8 * (c0 + c) + 4 * h, j, v[0], v[1]);
         }
       }
     }
@@ -343,7 +396,8 @@ __global__ __launch_bounds__(256) void k_gemm_n_fixup(GemmNArgs p, int R) {
   constexpr int Q = 4 * MT;
   const int wv = threadIdx.x >> 6, w = wv & 1, c = blockIdx.y * 2 + (wv >> 1);
   const int lane = threadIdx.x & 63, j = lane & 31, h = lane >> 5, tile = blockIdx.x;
-  if (8 * c >= p.M) return;
+  const int tm = (p.full + tile) % p.tiles_m, tn = (p.full + tile) / p.tiles_m;
+  if (32 * MT * tm + 8 * c >= p.M) return;
   const int b0 = share_of(tile * R, p.rem, p.nsk, R), b1 = share_of(tile * R + R - 1, p.rem, p.nsk, R);
   const float4* const slot = (const float4*)p.part + (size_t)share_piece(b0, tile, p.rem, p.nsk) * 4 * Q * 64 + lane;
   float v[2][4] = {};
@@ -355,26 +409,28 @@ __global__ __launch_bounds__(256) void k_gemm_n_fixup(GemmNArgs p, int R) {
 #pragma unroll
     for (int nb = 0; nb < 2; nb++) v[nb][0] += x[nb].x, v[nb][1] += x[nb].y, v[nb][2] += x[nb].z, v[nb][3] += x[nb].w;
   }
-  n_emit<MODE>(p, p.full + tile, w, 8 * c + 4 * h, j, v[0], v[1]);
+  n_emit<MODE>(p, tn, w, 32 * MT * tm + 8 * c + 4 * h, j, v[0], v[1]);
 }
 
 // ---- host side
 struct NPlan {
-  int MT, NKQ, form, full, rem, nsk;
+  int MT, NKQ, form, tiles_m, full, rem, nsk;
   double ns;
 };
 constexpr double kNSegment = 4000, kNFixup = 5000, kNBytesPerNs = 5000;
 // ns of a round: the MFMAs and dequant of NKQ units, or their weights at a CU's share of 6 TB/s
 static double n_round(int MT) { return MT == 4 ? 1650 : MT == 3 ? 1400 : MT == 2 ? 1150 : 900; }
 
-// affine: the decode GEMV's arithmetic (up to 64 rows)
-static NPlan n_plan(int M, int N, int K, bool affine) {
+// form: 0 dequantized weights, 1 the decode GEMV's arithmetic (up to 64 rows), 2 the same on int8 rows with scales per
+// 64-group (blocks of at most 64 rows)
+static NPlan n_plan(int M, int N, int K, int form) {
   NPlan pl{};
-  pl.MT = (M + 31) / 32;
+  pl.form = form;
+  pl.MT = form == 2 ? (M > 32 ? 2 : 1) : (M + 31) / 32;
+  pl.tiles_m = (M + 32 * pl.MT - 1) / (32 * pl.MT);
   const int G = K / kGroup, cu = cu_count();
   pl.NKQ = 4;
-  pl.form = affine;
-  const int R = G / pl.NKQ, tiles = (t64_bands(N) + 3) / 4, rem = tiles % cu;
+  const int R = G / pl.NKQ, tiles = pl.tiles_m * ((t64_bands(N) + 3) / 4), rem = tiles % cu;
   const double rd = n_round(pl.MT), whole = (tiles / cu) * (R * rd + kNSegment);
   pl.full = tiles;
   pl.ns = whole + (rem ? R * rd + kNSegment : 0);
@@ -392,8 +448,11 @@ bool gemm_n_applies(int M, int N, int K, int mode) {
   if (M <= 16 || M > 128 || K % 256 || t64_bytes(N, K) >= ((size_t)1 << 31)) return false;
   return mode != kModeSwiglu || N % 128 == 0;
 }
-size_t gemm_n_workspace(int M, int N, int K, bool affine) {
-  const NPlan pl = n_plan(M, N, K, affine);
+bool gemm_n_a8_applies(int M, int N, int K) {
+  return M > 16 && (size_t)M * K * 2 < ((size_t)1 << 31) && K % 256 == 0 && t64_bytes(N, K) < ((size_t)1 << 31);
+}
+size_t gemm_n_workspace(int M, int N, int K, int form) {
+  const NPlan pl = n_plan(M, N, K, form);
   return (size_t)share_pieces(pl.rem, pl.nsk) * n_slot_bytes(pl.MT);
 }
 
@@ -402,11 +461,11 @@ static int launch_n_mode(const GemmNArgs& a, hipStream_t st) {
   static bool attr = false;
   if (!attr) {
     (void)hipFuncSetAttribute((const void*)k_gemm_n<MT, NKQ, FORM, NS, MODE>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, n_lds(MT, NKQ));
+                              hipFuncAttributeMaxDynamicSharedMemorySize, n_lds(MT, NKQ, FORM));
     attr = true;
   }
   const int nblk = std::max(std::min(a.full, cu_count()), a.nsk);
-  hipLaunchKernelGGL((k_gemm_n<MT, NKQ, FORM, NS, MODE>), dim3(nblk), dim3(128 * NKQ), n_lds(MT, NKQ), st, a);
+  hipLaunchKernelGGL((k_gemm_n<MT, NKQ, FORM, NS, MODE>), dim3(nblk), dim3(128 * NKQ), n_lds(MT, NKQ, FORM), st, a);
   IFD_TRY(check_launch("gemm_n"));
   if (!a.rem) return IFD_OK;
   hipLaunchKernelGGL((k_gemm_n_fixup<MT, MODE>), dim3(a.rem, 2 * MT), dim3(256), 0, st, a, a.K / kGroup / NKQ);
@@ -422,18 +481,20 @@ static int launch_n_cfg(const GemmNArgs& a, hipStream_t st) {
   }
 }
 
-int launch_gemm_n(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
-                  bool affine, void* ws, size_t ws_bytes, hipStream_t st) {
+int launch_gemm_n(const uint16_t* A, int lda, const float* sxT, int Mp, const void* wt, int N, int K, void* C, int ldc,
+                  int M, int mode, int form, void* ws, size_t ws_bytes, hipStream_t st) {
   if (M == 0) return IFD_OK;
-  if ((size_t)M * lda * 2 >= ((size_t)1 << 31)) return fail(IFD_ERR_UNSUPPORTED, "gemm_n: operands past 2 GiB");
-  const NPlan pl = n_plan(M, N, K, affine);
-  const size_t need = gemm_n_workspace(M, N, K, affine);
+  if ((size_t)M * lda * 2 >= ((size_t)1 << 31) || (size_t)(K / kGroup) * Mp * 4 >= ((size_t)1 << 31))
+    return fail(IFD_ERR_UNSUPPORTED, "gemm_n: operands past 2 GiB");
+  const NPlan pl = n_plan(M, N, K, form);
+  const size_t need = gemm_n_workspace(M, N, K, form);
   if (need > ws_bytes || (need && !ws))
     return fail(IFD_ERR_WORKSPACE, "gemm_n needs %zu bytes of workspace, got %zu", need, ws_bytes);
-  GemmNArgs a{A, lda, (const uint8_t*)wt, (uint32_t)t64_bytes(N, K), N, K, C, ldc, M, mode, (float*)ws,
+  GemmNArgs a{A, lda, (const uint8_t*)wt, (uint32_t)t64_bytes(N, K), N, K, C, ldc, M, mode, sxT, Mp, pl.tiles_m, (float*)ws,
               N % 128 == 0 ? N / 64 : 0, pl.full, pl.rem, pl.nsk};
-  if (pl.MT == 1) return pl.form ? launch_n_cfg<1, 4, 1, 3>(a, st) : launch_n_cfg<1, 4, 0, 3>(a, st);
-  if (pl.MT == 2) return pl.form ? launch_n_cfg<2, 4, 1, 3>(a, st) : launch_n_cfg<2, 4, 0, 3>(a, st);
+  if (form == 2) return pl.MT == 1 ? launch_n_cfg<1, 4, 2, 3>(a, st) : launch_n_cfg<2, 4, 2, 3>(a, st);
+  if (pl.MT == 1) return form ? launch_n_cfg<1, 4, 1, 3>(a, st) : launch_n_cfg<1, 4, 0, 3>(a, st);
+  if (pl.MT == 2) return form ? launch_n_cfg<2, 4, 1, 3>(a, st) : launch_n_cfg<2, 4, 0, 3>(a, st);
   return pl.MT == 3 ? launch_n_cfg<3, 4, 0, 3>(a, st) : launch_n_cfg<4, 4, 0, 3>(a, st);
 }
 

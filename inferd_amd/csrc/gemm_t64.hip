@@ -362,7 +362,8 @@ static int launch_gemm_t_cfg(const GemmTArgs& p, int S, hipStream_t st) {
 // their row scales spill registers
 static GtPlan gemm_t_a8_plan(int M, int N, int K) { return gemm_t_plan(std::min(M, 64), N, K, M); }
 size_t gemm_t_a8_workspace(int M, int N, int K, int mode) {
-  return epilogue_ws_bytes(gemm_t_a8_plan(M, N, K).S, M, N, mode);
+  const size_t least = epilogue_ws_bytes(gemm_t_a8_plan(M, N, K).S, M, N, mode);
+  return gemm_n_a8_applies(M, N, K) ? std::max(gemm_n_workspace(M, N, K, 2), least) : least;
 }
 int launch_gemm_t_a8(const uint16_t* Ab, const float* sxT, int Mp, const void* wt, int N, int K, void* C, int ldc,
                      int M, int mode, void* ws, size_t ws_bytes, hipStream_t st) {
@@ -370,9 +371,11 @@ int launch_gemm_t_a8(const uint16_t* Ab, const float* sxT, int Mp, const void* w
   if (K % 128) return fail(IFD_ERR_ARG, "T64 W4A8 needs K %% 128 == 0 (K=%d)", K);
   if (mode == kModeSwiglu) return fail(IFD_ERR_UNSUPPORTED, "T64 W4A8: no SwiGLU mode");
   const GtPlan pl = gemm_t_a8_plan(M, N, K);
-  const size_t need = epilogue_ws_bytes(pl.S, M, N, mode);
+  const size_t need = gemm_t_a8_workspace(M, N, K, mode);
   if (need > ws_bytes || (need && !ws))
     return fail(IFD_ERR_WORKSPACE, "gemm_t64_w4a8 needs %zu bytes of workspace, got %zu", need, ws_bytes);
+  if (gemm_n_a8_applies(M, N, K))
+    return launch_gemm_n(Ab, K, sxT, Mp, wt, N, K, C, ldc, M, mode, 2, ws, ws_bytes, st);
   GemmTArgs p{Ab, K, (const uint8_t*)wt, N, K, C, ldc, M, mode, (float*)ws, pl.gps,
               (M + 32 * pl.MT - 1) / (32 * pl.MT), (t64_bands(N) + 4 * pl.NB - 1) / (4 * pl.NB), sxT, Mp};
   const int rc = pl.MT == 1 ? launch_gemm_t_cfg<1, 2, false, true>(p, pl.S, st)
@@ -392,7 +395,7 @@ int launch_gemm_t(const uint16_t* A, int lda, const void* wt, int N, int K, void
     if (need > ws_bytes || (need && !ws))
       return fail(IFD_ERR_WORKSPACE, "gemm_t64 needs %zu bytes of workspace, got %zu", need, ws_bytes);
     if (w) return launch_gemm_w(A, lda, wt, N, K, C, ldc, M, mode, ws, ws_bytes, st);
-    if (n) return launch_gemm_n(A, lda, wt, N, K, C, ldc, M, mode, gemm_n_affine(M, N, K, mode), ws, ws_bytes, st);
+    if (n) return launch_gemm_n(A, lda, nullptr, 0, wt, N, K, C, ldc, M, mode, gemm_n_affine(M, N, K, mode), ws, ws_bytes, st);
     const size_t plain = gemm_t_workspace(M, N, K, 0);
     uint16_t* gu = (uint16_t*)((char*)ws + align_up(plain, 256));
     IFD_TRY(launch_gemm_t(A, lda, wt, N, K, gu, N, M, 0, ws, plain, st));

@@ -75,12 +75,13 @@ bool gemm_w_applies(int M, int N, int K, int mode);
 size_t gemm_w_workspace(int M, int N, int K);
 int launch_gemm_w(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
                   void* ws, size_t ws_bytes, hipStream_t st);
-// GEMM on T64 weights for 16 < M <= 128 (gemm_n.hip), modes 0-2 and SwiGLU; affine: the decode GEMV's arithmetic
-// (up to 64 rows), else bf16-dequantized weights.
+// GEMM on T64 weights for 16 < M <= 128 (gemm_n.hip), modes 0-2 and SwiGLU. form: 0 bf16-dequantized weights, 1 the
+// decode GEMV's arithmetic (up to 64 rows), 2 the W4A8 of gemm_t_a8 below (A its bf16 integers, sxT their scales).
 bool gemm_n_applies(int M, int N, int K, int mode);
-size_t gemm_n_workspace(int M, int N, int K, bool affine);
-int launch_gemm_n(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
-                  bool affine, void* ws, size_t ws_bytes, hipStream_t st);
+bool gemm_n_a8_applies(int M, int N, int K);
+size_t gemm_n_workspace(int M, int N, int K, int form);
+int launch_gemm_n(const uint16_t* A, int lda, const float* sxT, int Mp, const void* wt, int N, int K, void* C, int ldc,
+                  int M, int mode, int form, void* ws, size_t ws_bytes, hipStream_t st);
 int launch_gemm_t(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
                   void* ws, size_t ws_bytes, hipStream_t st);
 // The stream-K plan (gemm_sk.hip) of a 4-bit shape: whether it has tiles for a third of the CUs (or one 128-row tile),

@@ -581,6 +581,26 @@ def test_gemm_t64_prefill_swiglu_bits(M, N, K):
     assert np.array_equal(g.host(ops.gemm_t64_swiglu(A, T)), g.host(ops.silu_mul(ops.gemm_t64(A, T))))
 
 
+@pytest.mark.parametrize("M,N,K,mode", [(17, 33, 256, 0), (33, 1000, 1280, 1), (64, 33024, 256, 2), (65, 640, 2048, 1),
+                                        (255, 4096, 768, 0)])
+def test_gemm_t64_w4a8_per_group_batches(M, N, K, mode):
+    """Per-group W4A8 past 16 rows: 32- and 64-row blocks (the last one partial), tiles whole and shared, odd widths, every
+    store mode, against the oracle on the GPU's own int8 rows."""
+    g, ops = _gu(), _ops()
+    codes, wq, s, b = gen.qlinear(N, K, seed=M + N + K)
+    T = ops.pack_t64(g.qlinear(wq, s, b))
+    A = gen.activations(M, K, seed=M + 3, row_scale=True)
+    C0 = gen.activations(M, N, seed=M + 4)
+    U, XS = orc.a8_quant(A, False)
+    outs = [g.host(ops.gemm_t64_w4a8(g.dev(U), g.dev(XS), T, g.dev(C0) if mode == 1 else None, mode=mode,
+                                     per_token=False)) for _ in range(2)]
+    assert np.array_equal(outs[0], outs[1])
+    rows = np.unique(np.r_[np.linspace(0, M - 1, 9).astype(int), M - 2])
+    Y = orc.w4a8(np.ascontiguousarray(U[rows]), np.ascontiguousarray(XS[rows]), wq, s, b)
+    ref = Y + gen.bf16_to_f32(C0[rows]) if mode == 1 else Y
+    gen.check_out(outs[0][rows], ref, 1e-4 if mode == 2 else 1e-2, (M, N, K, mode), fp32=mode == 2)
+
+
 @pytest.mark.parametrize("M,N,K,mode", [
     (17, 33, 256, 0),        # affine; one 128-column tile, two live bands (the second one column wide); one round of K
     (32, 1000, 2048, 1),     # shared tiles, N off the bands: neighbouring bands per tile
