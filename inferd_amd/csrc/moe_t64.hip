@@ -5,7 +5,7 @@
 //
 // Work items are (row tile, column tile) pairs: a row tile is up to BM = 32 MT sorted rows of one expert (the
 // dispatch's tile schedule), a column tile 8 bands (256 output columns; with SwiGLU 8 gate bands and the matching 8
-// up bands, 256 h columns). Items are numbered row tile-major, so an expert's column tiles are neighbours and share
+// up bands, 256 h columns; plain products of N % 512 == 0 take 16 bands, 512 columns). Items are numbered row tile-major, so an expert's column tiles are neighbours and share
 // its activation rows in L2. The grid is one block per CU; a block streams a contiguous run of (item, group pair)
 // units as one continuous sequence of (item, 64-group) steps, so the DMA pipeline runs across item boundaries without
 // draining. Without a piece buffer a run is whole items, [b n / nblk, (b + 1) n / nblk). With one (the balanced
@@ -15,7 +15,10 @@
 // is done; the last one sums the item's pieces in unit order and stores the item as a whole item ends. A cut item's
 // sum is therefore the sum of its K ranges' sums, in K order, and does not depend on timing.
 //
-// Block: 8 waves; wave w owns band w of the column tile (with SwiGLU, its gate band and its up band) over all MT M
+// Two kernels share this schedule: k_gqmm_v (16 waves, one band each, 32-row tiles with 16 bands per item) is described
+// at its code; k_gqmm_t takes 64-row tiles and plain items of 8 bands.
+//
+// k_gqmm_t's block: 8 waves; wave w owns band w of the column tile (with SwiGLU, its gate band and its up band) over all MT M
 // tiles. Two LDS rings filled by direct global -> LDS DMA: NA activation slabs [BM][64 bf16] (16-byte columns
 // XOR-swizzled by row pair), whose rows are gathered through perm by the DMA itself (row q of a tile is token
 // perm[q] / div, or row q of A), and NW weight stages (the item's code halves and (s, b) rows of one group). Waves
@@ -29,6 +32,7 @@
 // stores, rows past the segment at an out-of-range offset (dropped by the buffer bounds check).
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "common.h"
 #include "dma.h"
@@ -563,6 +567,323 @@ __global__ __launch_bounds__(kGqThreads, 1) void k_gqmm_t(GqArgs p) {
   }
 }
 
+// ---- the 16-wave kernel: 16 bands per item (SwiGLU: 8 gate bands and the matching 8 up bands; plain: 512 columns) ----
+// What bounds it: the expert stream from HBM, at 6 TB/s 0.79 us per CU and 64-group step of 16 bands. The 8-wave form
+// (two bands per wave, above) took 1.15 us: two waves per SIMD share its VALU at 2.4 to 3.5 cycles per instruction, and
+// every step opens with a barrier, the DMAs and their address arithmetic. Four waves per SIMD issue one per 1.7 to
+// 2.8 cycles, and a wave that owns one band needs no other wave's weights: they go straight to registers (LW group
+// pairs ahead; 3 measured 3% slower), LDS holds only the gathered activations, and one barrier serves a group pair.
+// Gate/up + SwiGLU at T = 100 (512 experts, H 2048, I 512, k = 10) 124 -> 115 us, down 70 -> 56 us; the MoE step 219 ->
+// 206 us, at T = 30 132 -> 125 us. A wave's sums run over K in order, the MFMA steps of k_gqmm, so that whole items keep
+// its bits.
+// Activations: NA chunks of two slabs [32][64 bf16] (16-byte columns XOR-swizzled by row pair); wave w < 8 gathers
+// rows 8 (w % 4) .. + 7 of slab w / 4 of a chunk. SwiGLU: wave w + 8 hands its bf16 up sums to wave w through
+// its own staging tile.
+constexpr int kGvNa = 6;
+constexpr size_t kGvLds = (size_t)kGvNa * 2 * gq_abytes(1) + 16 * kGqStg + 16;
+static_assert(kGvLds <= 160 * 1024 && 4 + (kGvNa - 2) * 5 <= 63, "LDS plan, vmcnt range");
+
+template <int K, int N, class F>
+__device__ __forceinline__ void gv_for(F&& f) {
+  if constexpr (K < N) {
+    f(std::integral_constant<int, K>{});
+    gv_for<K + 1, N>(f);
+  }
+}
+
+// AW: one of the waves that gather activations. BAL: a run may cut items (the balanced schedule).
+template <bool SILU, bool AW, bool BAL>
+__device__ __forceinline__ void gv_role(const GqArgs& p, uint8_t* lds, const int wave, const int b, const int nitems,
+                                        const int u0, const int u1) {
+  constexpr int NA = kGvNa, CH = 2 * gq_abytes(1), LW = 2, NS = LW + 1;  // NS register sets of one group pair
+  constexpr int D = AW ? 1 : 0;  // activation DMAs per pair
+  const int lane = threadIdx.x & 63, j = lane & 31, h = lane >> 5;
+  uint16_t* const stg = (uint16_t*)(lds + NA * CH + wave * kGqStg);
+  const int G2 = p.G / 2, nbands = t64_bands(p.N), n = u1 - u0;
+  const uint32_t gstride = (uint32_t)nbands * kT64Tile;
+
+  auto item_rows = [&](int item, int& e, int& c, int& q0, int& q1) __attribute__((always_inline)) {
+    const int tile = item >> p.nct_log2;
+    c = item & ((1 << p.nct_log2) - 1);
+    e = min(max(sload(p.tiles, 2 * tile), 0), p.E);
+    q0 = sload(p.tiles, 2 * tile + 1);
+    q1 = max(min(sload(p.offsets, e + 1), q0 + 32), q0 + 1);
+  };
+
+  // ---- the weight stream: this wave's band of the run's units in order, then staying on the last one
+  int w_item = u0 / G2, w_g2 = u0 - w_item * G2, w_left = n;
+  uint32_t wb_lo = 0, wb_hi = 0, w_so = 0;
+  auto open_w = [&]() __attribute__((always_inline)) {
+    const int tile = w_item >> p.nct_log2, c = w_item & ((1 << p.nct_log2) - 1);
+    const int e = min(max(sload(p.tiles, 2 * tile), 0), p.E);
+    // expert E is the shared expert; without one the reads stay inside the stack
+    const uint8_t* wb = e >= p.E && p.wsh ? p.wsh : p.wt + (size_t)min(e, p.E - 1) * p.ebytes;
+    wb_lo = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)wb);
+    wb_hi = __builtin_amdgcn_readfirstlane((uint32_t)((uintptr_t)wb >> 32));
+    const int band = SILU ? (wave < 8 ? 8 * c + wave : nbands / 2 + 8 * c + wave - 8) : 16 * c + wave;
+    w_so = (uint32_t)min(band, nbands - 1) * kT64Tile;
+  };
+  open_w();
+  w_so += (uint32_t)w_g2 * 2u * gstride;
+  u32x4 cw[NS][2];
+  uint32_t csb[NS][2];
+  auto load_w = [&](auto SC) __attribute__((always_inline)) {
+    constexpr int s = decltype(SC)::value;
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(((uint64_t)wb_hi << 32) | wb_lo), 0, (int)(uint32_t)p.ebytes, 0x00020000);
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      cw[s][k] = __builtin_amdgcn_raw_buffer_load_b128(r, 16 * lane, w_so + k * gstride, kNt);
+      csb[s][k] = __builtin_amdgcn_raw_buffer_load_b32(r, kT64Codes + 4 * j, w_so + k * gstride, kNt);
+    }
+    if (--w_left > 0) {
+      w_so += 2u * gstride;
+      if (++w_g2 == G2) {
+        w_g2 = 0, w_item++;
+        open_w();
+      }
+    }
+  };
+
+  // ---- the activation stream (AW): per-lane offsets of the item's rows, the pair's offset a scalar
+  int a_item = u0 / G2, a_g2 = u0 - a_item * G2, a_left = n, a_st = 0;
+  uint32_t voff = 0;
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)p.A, 0, (int)p.a_bytes, 0x00020000);
+  auto open_a = [&]() __attribute__((always_inline)) {
+    if constexpr (AW) {
+      int e, c, q0, q1;
+      item_rows(a_item, e, c, q0, q1);
+      const uint32_t rowb = 2u * (uint32_t)p.lda;
+      int v[8];
+#pragma unroll
+      for (int rho = 0; rho < 8; rho++) {
+        const int q = min(q0 + 8 * (wave & 3) + rho, q1 - 1);
+        v[rho] = p.perm ? sload(p.perm, q) : q;
+      }
+      if (p.perm && p.div_m)
+#pragma unroll
+        for (int rho = 0; rho < 8; rho++)
+          v[rho] = (int)__builtin_amdgcn_readfirstlane(__umulhi((uint32_t)v[rho], p.div_m));
+      int src = 0;
+#pragma unroll
+      for (int rho = 0; rho < 8; rho++) src = (lane >> 3) == rho ? v[rho] : src;
+      const int r = 8 * (wave & 3) + (lane >> 3);
+      voff = (uint32_t)src * rowb + 16u * (uint32_t)((lane & 7) ^ ((r >> 1) & 7)) + (wave >> 2) * 2u * kGroup;
+    }
+  };
+  auto issue_a = [&]() __attribute__((always_inline)) {
+    if constexpr (AW) {
+      uint8_t* const st = lds + a_st + (wave >> 2) * gq_abytes(1) + (wave & 3) * 1024;
+      bdma16(ra, st, voff, (uint32_t)a_g2 * 4u * kGroup);
+      a_st = a_st + CH == NA * CH ? 0 : a_st + CH;
+      if (--a_left > 0 && ++a_g2 == G2) {
+        a_g2 = 0, a_item++;
+        open_a();
+      }
+    }
+  };
+  open_a();
+
+  f32x16 acc = zero16();
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)p.C, 0, (int)p.c_bytes, 0x00020000);
+
+  // the item's outputs, through the waves' staging tiles [32][32] bf16; rows past the segment go
+  // to an offset past the buffer, which the bounds check drops. Every wave calls it (SwiGLU: block barriers inside).
+  auto epilogue = [&](int c, int q0, int q1) __attribute__((always_inline)) {
+    if (!SILU || wave >= 8)
+#pragma unroll
+      for (int r = 0; r < 16; r++) stg[(8 * (r / 4) + 4 * h + (r % 4)) * 32 + j] = f2bf(acc[r]);
+    if constexpr (SILU) {
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (wave < 8) {
+        const uint16_t* const up = stg + 8 * (kGqStg / 2);
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int o = (8 * (r / 4) + 4 * h + (r % 4)) * 32 + j;
+          stg[o] = f2bf(swiglu_f(bf2f(f2bf(acc[r])), bf2f(up[o])));
+        }
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the 16-byte reads below see the 2-byte writes (same wave)
+    if (!SILU || wave < 8) {
+      const int col = (SILU ? 8 * c + wave : 16 * c + wave) * 32 + 8 * (lane & 3);
+#pragma unroll
+      for (int s2 = 0; s2 < 2; s2++) {
+        const int row = 16 * s2 + (lane >> 2);
+        const u32x4 v = *(const u32x4*)(stg + row * 32 + 8 * (lane & 3));
+        const int q = q0 + row;
+        const int off = q < q1 ? (int)(((size_t)q * p.ldc + col) * 2) : 0x7FFFFFF0;
+        __builtin_amdgcn_raw_buffer_store_b128(v, rs, off, 0, 0);
+      }
+    }
+    if constexpr (SILU) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the up tile may be refilled
+    else asm volatile("" ::: "memory");
+    acc = zero16();
+  };
+  const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc((void*)p.part, 0, (int)p.part_bytes, 0x00020000);
+  auto piece_off = [&](int slot, int k4) __attribute__((always_inline)) {
+    return (int)((((size_t)slot * 16 + wave) * 4 + k4) * 64 + lane) * 16;
+  };
+
+  // prologue: the weights of LW pairs, the activations of NA - 1
+  gv_for<0, LW>([&](auto SC) __attribute__((always_inline)) { load_w(SC); });
+  for (int i = 0; i < NA - 1; i++) issue_a();
+  // (the waits of the loop count a steady stream: the prologue's chunks land first)
+  if constexpr (AW) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  int item = u0 / G2, ga = u0 - item * G2, left = min(G2 - ga, n), done = 0, rd = 0;
+  int ncut = 0, cut0 = 0, cut1 = 0;
+
+  // One group pair: its weights in set S. The barrier makes its chunk visible (each gathering wave first waits for its
+  // own DMAs of it: younger are those of NA - 2 pairs and their weights) and frees the chunk before.
+  auto pair = [&](auto SC) __attribute__((always_inline)) {
+    constexpr int S = decltype(SC)::value;
+    if constexpr (AW) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(4 + (NA - 2) * (D + 4)) : "memory");
+    else asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    issue_a();
+    load_w(std::integral_constant<int, (S + LW) % NS>{});
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const uint8_t* const st = lds + rd + k * gq_abytes(1);
+      const float s = bf2f((uint16_t)(csb[S][k] & 0xFFFFu)), bi = bf2f((uint16_t)(csb[S][k] >> 16));
+      const float sa = t64_sa(s), sb = t64_sb(s);
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        const u32x4 af = *(const u32x4*)(st + j * 128 + 16 * ((4 * h + t) ^ ((j >> 1) & 7)));
+        const u32x4 bf = t64_dequant(cw[S][k][t], sa, sb, bi);
+        acc = mfma_bf16(af, bf, acc);
+      }
+    }
+    rd = rd + CH == NA * CH ? 0 : rd + CH;
+    if (--left == 0) {  // the item's end, or the run's
+      int e, c, q0, q1;
+      item_rows(item, e, c, q0, q1);
+      (void)e;
+      done += min(G2 - ga, n - done);
+      if (!BAL || (ga == 0 && (u0 + done) % G2 == 0)) {
+        epilogue(c, q0, q1);
+      } else {
+        // a cut item's piece (slot 2 b for the run's first segment, 2 b + 1 for its last): the sums of its rows, written
+        // through to memory
+        const int slot = 2 * b + (item == u0 / G2 ? 0 : 1), nrows = q1 - q0;
+#pragma unroll
+        for (int k4 = 0; k4 < 4; k4++) {
+          if (8 * k4 + 4 * h >= nrows) continue;
+          const u32x4 v = {__float_as_uint(acc[4 * k4]), __float_as_uint(acc[4 * k4 + 1]),
+                           __float_as_uint(acc[4 * k4 + 2]), __float_as_uint(acc[4 * k4 + 3])};
+          __builtin_amdgcn_raw_buffer_store_b128(v, rp, piece_off(slot, k4), 0, kSc1);
+        }
+        if (ncut == 0) cut0 = item;
+        else cut1 = item;
+        ncut++;
+        acc = zero16();
+      }
+      item++, ga = 0, left = min(G2, n - done);
+    }
+  };
+  const int turns = n / NS, rest = n - turns * NS;
+#pragma clang loop unroll(disable)
+  for (int i = 0; i < turns; i++) gv_for<0, NS>([&](auto SC) __attribute__((always_inline)) { pair(SC); });
+  gv_for<0, NS - 1>([&](auto SC) __attribute__((always_inline)) {
+    if (SC.value < rest) pair(SC);
+  });
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no DMA lands in LDS after this; the pieces are in memory
+  if (!BAL || ncut == 0) return;
+
+  // arrivals at the cut items, one counter round trip for both: the last contributor of an item sums its pieces in
+  // unit order and stores it
+  const long U = (long)nitems * G2;
+  unsigned* const s_last = (unsigned*)(lds + NA * CH + 16 * kGqStg);
+  auto contributors = [&](int it, int& bf, int& bl) __attribute__((always_inline)) {
+    const long us = (long)it * G2;
+    bf = gq_block_of(us, p.nblk, U), bl = gq_block_of(us + G2 - 1, p.nblk, U);
+    int m = 0;
+    for (int bb = bf; bb <= bl; bb++) m += (long)(bb + 1) * U / p.nblk > (long)bb * U / p.nblk;
+    return m;
+  };
+  __syncthreads();  // every wave's pieces are complete
+  if (threadIdx.x == 0) {
+    unsigned old[2];
+#pragma unroll
+    for (int ci = 0; ci < 2; ci++)
+      if (ci < ncut) {
+        int bf, bl;
+        (void)contributors(ci == 0 ? cut0 : cut1, bf, bl);
+        old[ci] = __hip_atomic_fetch_add(p.cnt + bf, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+#pragma unroll
+    for (int ci = 0; ci < 2; ci++)
+      if (ci < ncut) {
+        int bf, bl;
+        const bool last = old[ci] + 1 == (unsigned)contributors(ci == 0 ? cut0 : cut1, bf, bl);
+        if (last) __hip_atomic_store(p.cnt + bf, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // next call
+        s_last[ci] = last;
+      }
+  }
+  __syncthreads();
+  const bool last0 = s_last[0] != 0, last1 = ncut > 1 && s_last[1] != 0;
+#pragma clang loop unroll(disable)
+  for (int r = ncut - 1; r >= 0; r--) {
+    if (!(r == 0 ? last0 : last1)) continue;
+    const int it = r == 0 ? cut0 : cut1;
+    int bf, bl;
+    (void)contributors(it, bf, bl);
+    const long lo_f = (long)bf * U / p.nblk, us = (long)it * G2;
+    int e, c, q0, q1;
+    item_rows(it, e, c, q0, q1);
+    (void)e;
+    const int nrows = q1 - q0;
+    constexpr int FB = 4;  // pieces whose loads are in flight together
+    for (int b0 = bf; b0 <= bl; b0 += FB) {
+      u32x4 v[FB][4];
+#pragma unroll
+      for (int z = 0; z < FB; z++) {
+        const int bb = b0 + z;
+        const bool has = bb <= bl && (long)(bb + 1) * U / p.nblk > (long)bb * U / p.nblk;
+        const int slot = bb == bf && lo_f < us ? 2 * bf + 1 : 2 * bb;
+#pragma unroll
+        for (int k4 = 0; k4 < 4; k4++)
+          v[z][k4] = has && 8 * k4 + 4 * h < nrows
+                         ? __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                         rp, piece_off(slot, k4), 0, kSc1))
+                         : u32x4{0u, 0u, 0u, 0u};
+      }
+#pragma unroll
+      for (int z = 0; z < FB; z++) {
+        const int bb = b0 + z;
+        if (bb > bl || (long)(bb + 1) * U / p.nblk <= (long)bb * U / p.nblk) continue;  // no piece
+#pragma unroll
+        for (int k4 = 0; k4 < 4; k4++)
+#pragma unroll
+          for (int x = 0; x < 4; x++) acc[4 * k4 + x] += __uint_as_float(v[z][k4][x]);
+      }
+    }
+    epilogue(c, q0, q1);  // stores the item and zeroes acc
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+template <bool SILU, bool BALK>
+__global__ __launch_bounds__(1024, 1) void k_gqmm_v(GqArgs p) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b = xcd_remap(blockIdx.x, p.nblk);
+  const int nitems = sload(p.ntiles, 0) << p.nct_log2;
+  const int G2 = p.G / 2;
+  int u0, u1;  // this block's run of (item, group pair) units, as k_gqmm_t's
+  const int per = (nitems + p.nblk - 1) / p.nblk;
+  const bool bal = BALK && p.part && (long)per * G2 * p.nblk - (long)nitems * G2 >= (long)kGqMinLoss * p.nblk;
+  if (bal) {
+    const long U = (long)nitems * G2;
+    u0 = (int)((long)b * U / p.nblk), u1 = (int)((long)(b + 1) * U / p.nblk);
+  } else {
+    u0 = (int)((long)b * nitems / p.nblk) * G2, u1 = (int)((long)(b + 1) * nitems / p.nblk) * G2;
+  }
+  if (u0 >= u1) return;  // block-uniform, before any barrier
+  if (wave < 8) gv_role<SILU, true, BALK>(p, lds, wave, b, nitems, u0, u1);
+  else gv_role<SILU, false, BALK>(p, lds, wave, b, nitems, u0, u1);
+}
+
 // ---- host side
 
 static int gq_cus() {
@@ -603,15 +924,32 @@ static double gq_expected_loss(int rows, int E, int tile_rows, int nct, int G2, 
   return std::ceil(n / nblk) * G2 - n * G2 / nblk;
 }
 
+template <bool SILU, bool BALK>
+static int launch_gv_kernel(const GqArgs& a, hipStream_t st) {
+  static bool attr = false;
+  if (!attr) {
+    (void)hipFuncSetAttribute((const void*)k_gqmm_v<SILU, BALK>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)kGvLds);
+    attr = true;
+  }
+  hipLaunchKernelGGL((k_gqmm_v<SILU, BALK>), dim3(a.nblk), dim3(1024), kGvLds, st, a);
+  return check_launch("moe_gather_qmm_t64");
+}
+
 template <int MT, bool SILU, bool WIDE>
 static int launch_gq_cfg(const GqArgs& a, int rows, hipStream_t st) {
   // the form compiled with the balanced schedule where the kernel is expected to take it (its whole-item path runs
   // slower there than in the form compiled without it); with fewer than kGqMinLoss group pairs per item no
   // whole-item run falls that far behind the even share
-  if (a.part && a.G / 2 >= kGqMinLoss &&
-      gq_expected_loss(rows, a.E + (a.wsh ? 1 : 0), 32 * MT, 1 << a.nct_log2, a.G / 2, a.nblk) >= kGqMinLoss - 2)
-    return launch_gq_kernel<MT, SILU, WIDE, true>(a, st);
-  return launch_gq_kernel<MT, SILU, WIDE, false>(a, st);
+  const bool bal =
+      a.part && a.G / 2 >= kGqMinLoss &&
+      gq_expected_loss(rows, a.E + (a.wsh ? 1 : 0), 32 * MT, 1 << a.nct_log2, a.G / 2, a.nblk) >= kGqMinLoss - 2;
+  // 32-row tiles with 16 bands per item: the 16-wave kernel. With 64 rows its sixteen waves would read each activation
+  // fragment from LDS once per band, 128 KB per step, which binds it (T = 500 over 128 experts 144 us against 140).
+  if constexpr (MT == 1 && (SILU || WIDE))
+    return bal ? launch_gv_kernel<SILU, true>(a, st) : launch_gv_kernel<SILU, false>(a, st);
+  else
+    return bal ? launch_gq_kernel<MT, SILU, WIDE, true>(a, st) : launch_gq_kernel<MT, SILU, WIDE, false>(a, st);
 }
 
 size_t moe_gather_t64_part_bytes(int tile_rows) { return 2 * (size_t)gq_cus() * gq_slot_bytes(tile_rows / 32); }
@@ -632,10 +970,9 @@ int launch_moe_gather_qmm_t64(const uint16_t* A, int lda, const int* perm, int d
   if (div < 1 || div > 64) return fail(IFD_ERR_ARG, "moe_gather_qmm_t64: div=%d must be in [1, 64]", div);
   // perm[q] / div as a multiply-high: exact for perm values below 2^32 / div (2^26 at div = 64)
   const uint32_t div_m = div == 1 ? 0u : (uint32_t)((((uint64_t)1 << 32) + div - 1) / div);
-  // plain products with output columns in whole 512-column tiles take the wide form (two bands per wave) on 64-row
-  // tiles; 32-row tiles (few rows per expert) keep 256-column items, twice as many, which spread more evenly over
-  // the CUs (config 4 at T = 128: 238 against 244 us, same box)
-  const bool wide = !silu && NO % 512 == 0 && tile_rows == 64;
+  // plain products with output columns in whole 512-column tiles take 512-column items (two bands per wave, or the
+  // 16-wave kernel)
+  const bool wide = !silu && NO % 512 == 0;
   const int nct = NO / (wide ? 512 : 256);
   if (nct & (nct - 1)) return fail(IFD_ERR_UNSUPPORTED, "moe_gather_qmm_t64: %d column tiles (not a power of 2)", nct);
   // every perm value is a routed slot below rows, so a sorted row reads one of the first (rows - 1) / div + 1 rows

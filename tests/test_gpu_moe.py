@@ -623,6 +623,30 @@ def test_gather_qmm_t64_bit_identical(T, E, H, I, k, tile_rows):
     assert np.array_equal(g.host(y_t), g.host(y_mlx)), "down"
 
 
+@pytest.mark.parametrize("K,N", [(128, 512), (256, 1024), (384, 512), (640, 2048), (1536, 512)])
+def test_gather_qmm_t64_one_band_per_wave(K, N):
+    """The 16-wave kernel (32-row tiles, 16 bands per item) over experts of 1, 31, 32, 33, 0 and 64 rows, with 1 to 12
+    group pairs per item (every remainder of its register sets): the bits of the MLX-layout gathered GEMM with whole
+    items and, on the items that it leaves whole, with the balanced schedule (it cuts all of those of 12 pairs)."""
+    g, ops = _gu(), _ops()
+    counts = [1, 31, 32, 33, 0, 64]
+    E, R = len(counts), sum(counts)
+    W = g.moew(*_stacks(K + N, E, K, N // 2)[0])
+    D = g.moew(*_stacks(K + N, E, N, K)[1])
+    x = g.dev(gen.activations(R, K, seed=K))
+    idx = g.dev(np.repeat(np.arange(E), counts).reshape(R, 1).astype(np.int32))
+    d32, dex = ops.moe_dispatch(idx, E), ops.moe_dispatch_ex(idx, E, 1, 32)
+    for stack, silu in ((W, True), (D, False)):
+        T = ops.pack_t64_stack(stack)
+        want = ops.moe_gather_qmm(x, d32[1], 1, d32, stack, silu=silu)
+        got = ops.moe_gather_qmm_t64(x, dex[1], 1, dex, T, silu=silu)
+        bal = ops.moe_gather_qmm_t64(x, dex[1], 1, dex, T, silu=silu, balanced=True)
+        torch.cuda.synchronize()
+        assert np.array_equal(g.host(got), g.host(want)), silu
+        ncut = _check_balanced(g, bal, got, dex, 32, 256 if silu else 512, K, f"silu={silu}")
+        assert (ncut > 0) == (K == 1536), ncut
+
+
 def _cut_items(nitems, G2, P, min_loss=8):
     """The items the balanced schedule cuts. It runs when whole-item runs would make the longest run at least
     min_loss (item, group pair) units longer than the even share; then block b runs units [b U / P, (b + 1) U / P) of
