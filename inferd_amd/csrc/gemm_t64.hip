@@ -316,6 +316,9 @@ static GtPlan gemm_t_plan(int M, int N, int K, int Mrows = 0) {
 // complement), as it always has; elsewhere the weights are rounded to bf16.
 static bool gemm_n_affine(int M, int N, int K, int mode) { return M <= 64 && !gemm_sk_applies(M, N, K, mode); }
 
+// At least a round of 256 x 256 tiles over 256 CUs.
+static bool tiles256_fill(int M, int N) { return (long)((M + 255) / 256) * ((t64_bands(N) + 7) / 8) >= 256; }
+
 // Past 16 rows a gate/up pair whose halves are no whole bands of the kernels below runs as the plain GEMM into the
 // workspace, then silu_mul.
 static bool swiglu_by_product(int M, int N, int K, int mode) {
@@ -326,18 +329,19 @@ static bool swiglu_by_product(int M, int N, int K, int mode) {
 size_t gemm_t_workspace(int M, int N, int K, int mode) {
   if (swiglu_by_product(M, N, K, mode))
     return align_up(gemm_t_workspace(M, N, K, 0), 256) + (size_t)M * N * sizeof(uint16_t);
-  // The size of a prefill shape decides which requests the static scratch of ifd_gemm_t64_noalloc serves, so it is never
-  // less than a split of 256-row tiles (from a round of them) or the stream-K kernel (below) would need.
-  if (gemm_w_applies(M, N, K, mode)) {
-    const long tiles = (long)((M + 255) / 256) * ((t64_bands(N) + 7) / 8), tail = tiles % 256;
-    size_t least = 0;
-    if (tiles < 256) least = gemm_sk_applies(M, N, K, mode) ? gemm_sk_workspace(M, N, K, mode) : 0;
-    else if (tail && tail <= 128) least = (size_t)std::min({256 / tail, 8L, K / kGroup / 4L}) * tail * 256 * 256 * 4;
-    return std::max(gemm_w_workspace(M, N, K), least);
+  const bool w = gemm_w_applies(M, N, K, mode), n = gemm_n_applies(M, N, K, mode);
+  // The size decides which requests the static scratch of ifd_gemm_t64_noalloc serves, so it is never less than a split
+  // of the last 256-row tiles (from a round of them), the stream-K kernel or the K split would need.
+  size_t least = 0;
+  if ((w || n) && tiles256_fill(M, N)) {
+    const long tail = (long)((M + 255) / 256) * ((t64_bands(N) + 7) / 8) % 256;
+    if (tail && tail <= 128) least = (size_t)std::min({256 / tail, 8L, K / kGroup / 4L}) * tail * 256 * 256 * 4;
+  } else {
+    least = gemm_sk_applies(M, N, K, mode) ? gemm_sk_workspace(M, N, K, mode)
+                                           : epilogue_ws_bytes(gemm_t_plan(M, N, K).S, M, N, mode);
   }
-  const size_t least =
-      gemm_sk_applies(M, N, K, mode) ? gemm_sk_workspace(M, N, K, mode) : epilogue_ws_bytes(gemm_t_plan(M, N, K).S, M, N, mode);
-  return gemm_n_applies(M, N, K, mode) ? std::max(gemm_n_workspace(M, N, K, gemm_n_affine(M, N, K, mode)), least) : least;
+  if (w) return std::max(gemm_w_workspace(M, N, K), least);
+  return n ? std::max(gemm_n_workspace(M, N, K, gemm_n_affine(M, N, K, mode)), least) : least;
 }
 
 template <int MT, int NB, bool DEQ, bool A8 = false>
@@ -388,8 +392,11 @@ int launch_gemm_t(const uint16_t* A, int lda, const void* wt, int N, int K, void
                   void* ws, size_t ws_bytes, hipStream_t st) {
   if (M == 0) return IFD_OK;
   if (K % 128) return fail(IFD_ERR_ARG, "T64 GEMM needs K %% 128 == 0 (K=%d)", K);
-  const bool by_product = swiglu_by_product(M, N, K, mode);
-  const bool w = gemm_w_applies(M, N, K, mode), n = gemm_n_applies(M, N, K, mode);
+  // activations past a buffer's 2 GiB (a large row stride): the K split, which addresses them by pointer, takes them
+  // at shapes below the stream-K rule, as it always has; gemm_w.hip and gemm_n.hip refuse them
+  const bool far = (size_t)M * lda * 2 >= ((size_t)1 << 31) && !tiles256_fill(M, N) && !gemm_sk_applies(M, N, K, mode);
+  const bool by_product = !far && swiglu_by_product(M, N, K, mode);
+  const bool w = !far && gemm_w_applies(M, N, K, mode), n = !far && gemm_n_applies(M, N, K, mode);
   if (by_product || w || n) {
     const size_t need = gemm_t_workspace(M, N, K, mode);
     if (need > ws_bytes || (need && !ws))

@@ -241,3 +241,9 @@ def test_moe_rows_checks():
     assert call64(T=0) == _lib.IFD_OK
     assert call64() == _lib.IFD_ERR_WORKSPACE
     assert call64(sw=4096, ys=None) == _lib.IFD_ERR_WORKSPACE
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 151936, 5120), (64, 151936, 5120), (128, 248320, 5120), (300, 34816, 5120)])
+def test_noalloc_scratch_serves_wide_linears(M, N, K):
+    """A head over a whole vocabulary, or a wide layer, fits the static scratch of ifd_gemm_t64_noalloc."""
+    assert _lib.lib().ifd_gemm_t64_workspace(M, N, K) <= 68 << 20  # IFD_NOALLOC_SCRATCH_BYTES
