@@ -1,10 +1,10 @@
 // Stream-K GEMM on T64x8 (8-bit) weights past the decode GEMV's rows: C (mode) = A . W^T with every weight dequantized
 // to bf16(s q + b) (MLX 8-bit qmm rounding, third_party/mlx/.../quantized.h:528-535) and fp32 accumulation. Serves the
 // reference's affine_qmm_t_nax (quantized_nax.h:938-1076) with its split-K variant
-// (engine/kernels/qmm_splitk.metal:14-107) at BITS = 8. (The BITS = 4 form served T64 decode batches; gemm_n.hip does.)
+// (engine/kernels/qmm_splitk.metal:14-107).
 //
 // Work is the set of units (tile, 64-group); a tile is BM = 32 MT rows x 8 bands (256 columns). Block b (of nblk,
-// one or two per CU) takes units [b U / nblk, (b + 1) U / nblk) (stream-K): every CU streams the same weight bytes
+// one per CU) takes units [b U / nblk, (b + 1) U / nblk) (stream-K): every CU streams the same weight bytes
 // whatever the tile count. A run never covers more than one tile's worth of groups, so it touches at most two tiles
 // ("segments"). A segment covering its whole tile is stored by the block; any other segment is a piece of its tile,
 // and its fp32 sums go to the block's partial slot (the first segment's as soon as it ends, while the run goes on).
@@ -44,27 +44,19 @@ constexpr int kSkThreads = 64 * kSkWaves;
 constexpr int kSkLds = 160 * 1024;  // LDS per CU
 constexpr int kSkRow = 256 + 4;  // staged tile row stride (floats): rows h = 0, 1 of one store fall in other banks
 
-// BITS = 4: T64 weights; BITS = 8: T64x8 weights (t64.h), whose code tiles are twice as large (two 1 KB halves per
-// band and group, each one DMA) and are dequantized from the stored q - 128 bytes.
-__host__ __device__ constexpr int sk_codes(int BITS) { return BITS == 8 ? kT64x8Codes : kT64Codes; }
-__host__ __device__ constexpr int sk_tileb(int BITS) { return BITS == 8 ? kT64x8Tile : kT64Tile; }
+// T64x8 weights (t64.h): the code tiles are two 1 KB halves per band and group, each one DMA.
 // weights of a stage: 8 bands' codes + 8 (s, b) rows
-__host__ __device__ constexpr int sk_wbytes(int BITS) { return 8 * sk_codes(BITS) + 8 * 128; }
+__host__ __device__ constexpr int sk_wbytes() { return 8 * kT64x8Codes + 8 * 128; }
 
-// 4-bit 32-row tiles run two blocks per CU (two waves per SIMD hide the latency of their short steps), other tiles
-// one (an 8-bit stage is too large for two rings of four). A stage holds one step's activation slab and weights; the
-// ring is as deep as LDS allows, at most 8 stages.
-__host__ __device__ constexpr int sk_bpc(int MT, int BITS) { return MT == 1 && BITS == 4 ? 2 : 1; }
 __host__ __device__ constexpr int sk_abytes(int MT) { return MT * 32 * 128; }
-__host__ __device__ constexpr int sk_stage(int MT, int BITS) { return sk_abytes(MT) + sk_wbytes(BITS); }
-__host__ __device__ constexpr int sk_ring(int MT, int BITS) {
-  return (kSkLds / sk_bpc(MT, BITS) - 64) / sk_stage(MT, BITS) < 8 ? (kSkLds / sk_bpc(MT, BITS) - 64) / sk_stage(MT, BITS)
-                                                                   : 8;
+__host__ __device__ constexpr int sk_stage(int MT) { return sk_abytes(MT) + sk_wbytes(); }
+__host__ __device__ constexpr int sk_ring(int MT) {
+  return (kSkLds - 64) / sk_stage(MT) < 8 ? (kSkLds - 64) / sk_stage(MT) : 8;
 }
 // the ring, and after the K loop the staged tile [32 MT][kSkRow] fp32 in the same memory
-__host__ __device__ constexpr size_t sk_lds(int MT, int BITS) {
-  return (size_t)sk_ring(MT, BITS) * sk_stage(MT, BITS) > (size_t)MT * 32 * kSkRow * 4
-             ? (size_t)sk_ring(MT, BITS) * sk_stage(MT, BITS)
+__host__ __device__ constexpr size_t sk_lds(int MT) {
+  return (size_t)sk_ring(MT) * sk_stage(MT) > (size_t)MT * 32 * kSkRow * 4
+             ? (size_t)sk_ring(MT) * sk_stage(MT)
              : (size_t)MT * 32 * kSkRow * 4;
 }
 
@@ -121,12 +113,12 @@ __device__ __forceinline__ void sk_static_for(F&& f) {
 // register set is a compile-time constant; a run enters it at its phase (Duff's device). A step issues about 220
 // instructions for its 8 MT MFMAs, which a single wave per SIMD issues one every ~4 cycles: the stream's bookkeeping
 // is a few scalar adds and one countdown per step.
-template <int MT, int BITS>
+template <int MT>
 __device__ __forceinline__ void sk_body(const GemmSkArgs& p, uint8_t* lds, const int wave, const int b) {
-  constexpr int BM = 32 * MT, R = sk_ring(MT, BITS), A_BYTES = sk_abytes(MT), STAGE = sk_stage(MT, BITS);
-  constexpr int CODES = sk_codes(BITS), TILEB = sk_tileb(BITS);
+  constexpr int BM = 32 * MT, R = sk_ring(MT), A_BYTES = sk_abytes(MT), STAGE = sk_stage(MT);
+  constexpr int CODES = kT64x8Codes, TILEB = kT64x8Tile;
   constexpr int NE = MT * 16;             // accumulators per lane and band
-  constexpr int NH = BITS / 4;            // 1 KB code DMAs per band
+  constexpr int NH = 2;            // 1 KB code DMAs per band
   constexpr int NWC = 2 * NH;             // code DMAs per pair (two bands)
   constexpr int PAIR = MT + NWC + 1;      // DMAs per pair: activation rows, codes, the (s, b) rows
   constexpr int UNR = R % 2 ? 2 * R : R;  // steps per unrolled body
@@ -213,30 +205,23 @@ __device__ __forceinline__ void sk_body(const GemmSkArgs& p, uint8_t* lds, const
       cd.sb[nb] = *(const uint32_t*)(wst + 8 * CODES + band * 128 + 4 * j);
     }
   };
-  // MFMA step t's B fragment of band nb: column j, k = 32 h + 8 t .. + 7 dequantized to bf16(s q + b). sa, sbs: the
-  // scalings of s for t64_dequant (4 bits); 8 bits: sa = s, and q = stored byte ^ 0x80.
-  auto deq_step = [&](const Codes& cd, int nb, int t, float sa, float sbs, float bi) __attribute__((always_inline)) {
-    if constexpr (BITS == 4) {
-      return t64_dequant(cd.w[nb][0][t], sa, sbs, bi);
-    } else {
-      (void)sbs;
-      return dequant8x8_bf16(cd.w[nb][t / 2][2 * (t % 2)] ^ 0x80808080u, cd.w[nb][t / 2][2 * (t % 2) + 1] ^ 0x80808080u,
-                             sa, bi);
-    }
+  // MFMA step t's B fragment of band nb: column j, k = 32 h + 8 t .. + 7 dequantized to bf16(s q + b), q = stored
+  // byte ^ 0x80.
+  auto deq_step = [&](const Codes& cd, int nb, int t, float sc, float bi) __attribute__((always_inline)) {
+    return dequant8x8_bf16(cd.w[nb][t / 2][2 * (t % 2)] ^ 0x80808080u, cd.w[nb][t / 2][2 * (t % 2) + 1] ^ 0x80808080u,
+                           sc, bi);
   };
-  auto scales = [&](uint32_t sbw, float& sa, float& sbs, float& bi) __attribute__((always_inline)) {
-    const float sc = bf2f((uint16_t)(sbw & 0xFFFFu));
+  auto scales = [&](uint32_t sbw, float& sc, float& bi) __attribute__((always_inline)) {
+    sc = bf2f((uint16_t)(sbw & 0xFFFFu));
     bi = bf2f((uint16_t)(sbw >> 16));
-    sa = BITS == 4 ? t64_sa(sc) : sc;
-    sbs = BITS == 4 ? t64_sb(sc) : 0.f;
   };
   auto dequant = [&](const Codes& cd, u32x4 (&bf)[2][4]) __attribute__((always_inline)) {
 #pragma unroll
     for (int nb = 0; nb < 2; nb++) {
-      float sa, sbs, bi;
-      scales(cd.sb[nb], sa, sbs, bi);
+      float sc, bi;
+      scales(cd.sb[nb], sc, bi);
 #pragma unroll
-      for (int t = 0; t < 4; t++) bf[nb][t] = deq_step(cd, nb, t, sa, sbs, bi);
+      for (int t = 0; t < 4; t++) bf[nb][t] = deq_step(cd, nb, t, sc, bi);
     }
   };
   // activation fragments of stage s: M tile a, MFMA step t takes k = 32 h + 8 t .. + 7 (logical column 4 h + t)
@@ -280,13 +265,13 @@ __device__ __forceinline__ void sk_body(const GemmSkArgs& p, uint8_t* lds, const
   // in its shadow.
   auto step = [&](auto KC) __attribute__((always_inline)) {
     constexpr int K = decltype(KC)::value, S = K % R, P = K % 2, S1 = (S + 1) % R, S2 = (S + 2) % R;
-    constexpr int NDS = 4 * MT + 2 * (NH + 1), DEQ = BITS == 4 ? 17 : 22;
+    constexpr int NDS = 4 * MT + 2 * (NH + 1), DEQ = 22;
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((R - 3) * PAIR) : "memory");
     const uint8_t* const ast = lds + S1 * STAGE;           // activation fragments of step i + 1
     const uint8_t* const wst = lds + S2 * STAGE + A_BYTES;  // codes of step i + 2
-    float sa[2], sbs[2], bi[2];
+    float sc[2], bi[2];
 #pragma unroll
-    for (int nb = 0; nb < 2; nb++) scales(cd[P].sb[nb], sa[nb], sbs[nb], bi[nb]);
+    for (int nb = 0; nb < 2; nb++) scales(cd[P].sb[nb], sc[nb], bi[nb]);
 #pragma unroll
     for (int g = 0; g < 8; g++) {
 #pragma unroll
@@ -302,7 +287,7 @@ __device__ __forceinline__ void sk_body(const GemmSkArgs& p, uint8_t* lds, const
           else cd[P ^ 1].sb[nb] = *(const uint32_t*)(wst + 8 * CODES + band * 128 + 4 * j);
         }
       }
-      bf[P ^ 1][g / 4][g % 4] = deq_step(cd[P], g / 4, g % 4, sa[g / 4], sbs[g / 4], bi[g / 4]);
+      bf[P ^ 1][g / 4][g % 4] = deq_step(cd[P], g / 4, g % 4, sc[g / 4], bi[g / 4]);
 #pragma unroll
       for (int m = g * MT; m < (g + 1) * MT; m++) {
         const int am = m % MT, nb = (m / MT) % 2, t = m / (2 * MT);
@@ -431,13 +416,13 @@ __device__ __forceinline__ void sk_body(const GemmSkArgs& p, uint8_t* lds, const
   write_slot(2 * b + (two ? 1 : 0));  // a piece of a cut tile: k_sk_fixup sums the pieces
 }
 
-template <int MT, int BITS>
-__global__ __launch_bounds__(kSkThreads, sk_bpc(MT, BITS)) void k_gemm_sk(GemmSkArgs p) {
-  static_assert(sk_lds(MT, BITS) + 64 <= kSkLds / sk_bpc(MT, BITS), "LDS plan");
+template <int MT>
+__global__ __launch_bounds__(kSkThreads, 1) void k_gemm_sk(GemmSkArgs p) {
+  static_assert(sk_lds(MT) + 64 <= kSkLds, "LDS plan");
   extern __shared__ __align__(16) uint8_t lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int b = xcd_remap(blockIdx.x, p.nblk);
-  sk_body<MT, BITS>(p, lds, wave, b);
+  sk_body<MT>(p, lds, wave, b);
 }
 
 // Sum of a cut tile's pieces (partial slots, in unit order) and its store. Block (tile, w, a), wave q: the float4
@@ -518,7 +503,7 @@ struct SkPlan {
 static SkPlan gemm_sk_plan(int M, int N, int K, int bits = 4) {
   SkPlan pl{};
   pl.MT = M <= 32 ? 1 : M <= 64 ? 2 : 4;
-  const int bpc = pl.MT == 1 && bits == 4 ? 2 : 1;  // sk_bpc
+  const int bpc = pl.MT == 1 && bits == 4 ? 2 : 1;  // the 4-bit plan of 32-row tiles had two blocks per CU
   pl.tiles_m = (M + 32 * pl.MT - 1) / (32 * pl.MT);
   pl.tiles_n = (t64_bands(N) + 7) / 8;
   pl.G = K / kGroup;
@@ -552,15 +537,15 @@ size_t gemm_sk_workspace(int M, int N, int K, int mode) {
 
 size_t gemm_sk8_workspace(int M, int N, int K) { return sk_part_bytes(gemm_sk_plan(M, N, K, 8)); }
 
-template <int MT, int BITS>
+template <int MT>
 static int launch_sk_cfg(const GemmSkArgs& a, bool fixup, hipStream_t st) {
-  constexpr size_t lds = sk_lds(MT, BITS);
+  constexpr size_t lds = sk_lds(MT);
   static bool attr = false;
   if (!attr) {
-    (void)hipFuncSetAttribute((const void*)k_gemm_sk<MT, BITS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    (void)hipFuncSetAttribute((const void*)k_gemm_sk<MT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     attr = true;
   }
-  hipLaunchKernelGGL((k_gemm_sk<MT, BITS>), dim3(a.nblk), dim3(kSkThreads), lds, st, a);
+  hipLaunchKernelGGL((k_gemm_sk<MT>), dim3(a.nblk), dim3(kSkThreads), lds, st, a);
   IFD_TRY(check_launch("gemm_sk"));
   if (!fixup) return IFD_OK;
   hipLaunchKernelGGL(k_sk_fixup<MT>, dim3(a.ntiles, a.swi ? 4 : 8, MT), dim3(256), 0, st, a);
@@ -578,11 +563,10 @@ int launch_sk_fixup_rows(const float* part, int tiles_m, int tiles_n, int tile0,
   return check_launch("sk fixup");
 }
 
-template <int BITS>
-static int launch_sk_bits(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
-                          void* ws, size_t ws_bytes, hipStream_t st) {
-  const SkPlan pl = gemm_sk_plan(M, N, K, BITS);
-  const size_t need = sk_part_bytes(pl), wbytes = BITS == 8 ? t64x8_bytes(N, K) : t64_bytes(N, K);
+static int launch_sk(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
+                     void* ws, size_t ws_bytes, hipStream_t st) {
+  const SkPlan pl = gemm_sk_plan(M, N, K, 8);
+  const size_t need = sk_part_bytes(pl), wbytes = t64x8_bytes(N, K);
   if (need > ws_bytes || !ws)
     return fail(IFD_ERR_WORKSPACE, "gemm_sk needs %zu bytes of workspace, got %zu", need, ws_bytes);
   if (need >= (size_t)1 << 31) return fail(IFD_ERR_UNSUPPORTED, "gemm_sk: partials past 2 GiB");
@@ -597,9 +581,9 @@ static int launch_sk_bits(const uint16_t* A, int lda, const void* wt, int N, int
     fixup = sk_block_of(t * pl.G + pl.G - 1, pl.nblk, U) != sk_block_of(t * pl.G, pl.nblk, U);
   GemmSkArgs a{A, lda, (const uint8_t*)wt, (uint32_t)wbytes, N, K, C, ldc, M, mode, (float*)ws, (uint32_t)need,
                pl.tiles_m, pl.tiles_n, pl.G, pl.nblk, mode == kModeSwiglu ? N / 64 : 0, 0, (int)tiles, nullptr, 0, 0};
-  if (pl.MT == 1) return launch_sk_cfg<1, BITS>(a, fixup, st);
-  if (pl.MT == 2) return launch_sk_cfg<2, BITS>(a, fixup, st);
-  return launch_sk_cfg<4, BITS>(a, fixup, st);
+  if (pl.MT == 1) return launch_sk_cfg<1>(a, fixup, st);
+  if (pl.MT == 2) return launch_sk_cfg<2>(a, fixup, st);
+  return launch_sk_cfg<4>(a, fixup, st);
 }
 
 int launch_gemm_sk8(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
@@ -607,7 +591,7 @@ int launch_gemm_sk8(const uint16_t* A, int lda, const void* wt, int N, int K, vo
   if (M == 0) return IFD_OK;
   if (K % kGroup || (mode == kModeSwiglu && N % 256))
     return fail(IFD_ERR_UNSUPPORTED, "gemm_sk8: shape N=%d K=%d", N, K);
-  return launch_sk_bits<8>(A, lda, wt, N, K, C, ldc, M, mode, ws, ws_bytes, st);
+  return launch_sk(A, lda, wt, N, K, C, ldc, M, mode, ws, ws_bytes, st);
 }
 
 }  // namespace ifd
