@@ -487,8 +487,8 @@ def main():
         "data": "synthetic (seeded 4-bit affine weights, bf16 N(0,1) activations)",
     }
     # HBM bytes per call of a bench call, from the FETCH_SIZE / WRITE_SIZE counter runs of the same workload scaled by
-    # a plain 256 MiB device copy (profiles/traffic_c1_c0_c4.md); calls not measured report null
-    measured_traffic = {"gate_up_swiglu_M128": 216816249}
+    # a plain 256 MiB device copy (profiles/perf_cases.md); calls not measured report null
+    measured_traffic = {"gate_up_swiglu_M128": 146664177}
 
     def roofline(d):
         # the bound is the larger of the call's two floors: its algorithmic bytes at HBM peak, its flops at dense

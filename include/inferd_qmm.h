@@ -152,7 +152,7 @@ int ifd_gemm_t64_noalloc(const void* A, int lda, const void* wt, int N, int K, v
                          void* stream);
 /* Gate/up projection with its SwiGLU: W (T64) holds [gate (N/2) | up (N/2)] rows and H [M][N/2] (row stride ldh)
  * receives silu_mul of the bf16 product: bit-identical to ifd_gemm_t64 (mode 0) followed by ifd_silu_mul for
- * M <= 16 and for M > 128 with N % 256 == 0; on the stream-K rows between, the fused tiles cut K at other places than the
+ * M <= 16 and for M > 128 with N % 256 == 0; on the rows between, the fused tiles may cut K at other places than the
  * plain GEMM's, so a gate or up sum may differ from it by one bf16 step before the SwiGLU. Replaces
  * the reference's gemm + silu_mul pair (qwen35.h:1910-1912, shared expert; qwen35.h:2868-2878, dense MLP) with one
  * call that never stores the [M][N] product when K is split (the SwiGLU runs in the split-K reduction).

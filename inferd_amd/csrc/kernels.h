@@ -120,7 +120,7 @@ int launch_qmv_t_multi(const uint16_t* A, int lda, int n, const void* const* wts
                        hipStream_t st);
 // W4A8 with per-(row, 64-group) int8 activations on T64 weights, in the affine bf16-MFMA form (xq as exact bf16
 // integers): the prep writes Ab = bf16(U) [M][K] and sxT = sx transposed [G][Mp] (zero past M); M <= 16 runs the
-// decode GEMV (qmv_t_workspace(M, N, K, mode)), more rows the affine k_gemm_t (gemm_t_a8_workspace).
+// decode GEMV (qmv_t_workspace(M, N, K, mode)), more rows k_gemm_n (form 2) (gemm_t_a8_workspace).
 int w4a8g_mp(int M);
 int launch_w4a8g_prep(const int8_t* U, const float* XS, int M, int K, uint16_t* Ab, float* sxT, int Mp, hipStream_t st);
 int launch_qmv_t_a8(const uint16_t* Ab, const float* XS, const void* wt, int N, int K, void* C, int ldc, int M,
