@@ -220,7 +220,9 @@ __global__ __launch_bounds__(128 * NKQ, 1) void k_gemm_n(GemmNArgs p) {
     uint32_t w3[2];
     float sa[2], sb[2], bi[2];
 
-    // prologue, after the weights': A(0 .. RA - 2) and half of A(RA - 1)
+    // prologue, after the weights': A(0 .. RA - 2) and half of A(RA - 1). All but the half land before the first unit:
+    // the count of the units' wait (below) is that of a stream with weights between the slabs, which begins here, so
+    // it covers the slabs that the units issue (from A(RA - 1)) and not these.
 #pragma unroll
     for (int s = 0; s < RA; s++) {
 #pragma unroll
@@ -230,7 +232,7 @@ __global__ __launch_bounds__(128 * NKQ, 1) void k_gemm_n(GemmNArgs p) {
         adv_a();
       }
     }
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((RA - 2) * (2 * MT + SX) + MT) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(MT) : "memory");
 #pragma unroll
     for (int a = 0; a < MT; a++) af[a] = *(const u32x4*)(ring + asw + a * 4096);
     auto scales = [&](uint32_t x, int nb) __attribute__((always_inline)) {
@@ -263,7 +265,8 @@ __global__ __launch_bounds__(128 * NKQ, 1) void k_gemm_n(GemmNArgs p) {
 #pragma unroll
           for (int nb = 0; nb < 2; nb++) scales(csb[S1][nb], nb), w3[nb] = cw[S1][nb][3];
         if (k == 1) load_w(std::integral_constant<int, FORM == 0 ? S : SL>{});
-        // A(i + 1) has landed: younger are A(i + 2 .. i + RA - 1) and the weights of RA - 1 units
+        // A(i + 1) has landed: in the prologue (i + 1 < RA - 1), or else, its second half being unit i + 2 - RA's, younger
+        // are A(i + 2 .. i + RA - 1) and the weights of units i + 2 - RA .. i
         if (k == 3)
           asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((RA - 1) * 4 + (RA - 2) * (2 * MT + SX)) : "memory");
         const uint8_t* const src = ring + ((asw ^ (16u * ((k + 1) & 3))) + (k == 3 ? sln : sl));
