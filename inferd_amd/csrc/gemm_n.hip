@@ -254,7 +254,10 @@ __global__ __launch_bounds__(128 * NKQ, 1) void k_gemm_n(GemmNArgs p) {
     // the comment of each: the second half of A(i + RA - 1) (k = 0), W(i + NS) or, FORM 1, W(i + NS - 1) into the
     // registers of W(i) or W(i - 1) (k = 1), the first half of A(i + RA) (k = 3, into the slab whose last fragments were read at k = 2).
     int sl = 0, slp = (RA - 1) * AB, sln = AB, xr = 0, xw = (RA - 1) * 256;
-    auto unit = [&](auto SC) __attribute__((always_inline)) {
+    // TAIL: one of the segment's last units, past the whole turns of the register sets. Nothing reads what it would load
+    // (the compiler may drop such a load, and the count with it), so it loads no weights and its wait counts none.
+    auto unit = [&](auto SC, auto TAIL) __attribute__((always_inline)) {
+      constexpr int YOUNGER = (RA - 2) * (2 * MT + SX) + (TAIL.value ? 0 : (RA - 1) * 4);
       constexpr int S = decltype(SC)::value, S1 = (S + 1) % NS, SL = (S + NS - 1) % NS;
       if constexpr (FORM != 0)
 #pragma unroll
@@ -264,11 +267,11 @@ __global__ __launch_bounds__(128 * NKQ, 1) void k_gemm_n(GemmNArgs p) {
         if (FORM == 0 && k == 1)
 #pragma unroll
           for (int nb = 0; nb < 2; nb++) scales(csb[S1][nb], nb), w3[nb] = cw[S1][nb][3];
-        if (k == 1) load_w(std::integral_constant<int, FORM == 0 ? S : SL>{});
+        if (k == 1 && !TAIL.value) load_w(std::integral_constant<int, FORM == 0 ? S : SL>{});
         // A(i + 1) has landed: in the prologue (i + 1 < RA - 1), or else, its second half being unit i + 2 - RA's, younger
         // are A(i + 2 .. i + RA - 1) and the weights of units i + 2 - RA .. i
         if (k == 3)
-          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((RA - 1) * 4 + (RA - 2) * (2 * MT + SX)) : "memory");
+          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(YOUNGER) : "memory");
         const uint8_t* const src = ring + ((asw ^ (16u * ((k + 1) & 3))) + (k == 3 ? sln : sl));
         const int kw = (k + 3) & 3;
         if constexpr (FORM != 0)
@@ -343,9 +346,10 @@ __global__ __launch_bounds__(128 * NKQ, 1) void k_gemm_n(GemmNArgs p) {
     // without exits in its middle)
     const int turns = nr / NS, rest = nr - turns * NS;
 #pragma clang loop unroll(disable)
-    for (int i = 0; i < turns; i++) static_for<0, NS>([&](auto SC) __attribute__((always_inline)) { unit(SC); });
+    for (int i = 0; i < turns; i++)
+      static_for<0, NS>([&](auto SC) __attribute__((always_inline)) { unit(SC, std::false_type{}); });
     static_for<0, NS - 1>([&](auto SC) __attribute__((always_inline)) {
-      if (SC.value < rest) unit(SC);
+      if (SC.value < rest) unit(SC, std::true_type{});
     });
 
     // ---- the K-groups' sums meet in LDS, PQ quads of rows (quad c: rows 8 c + 4 h .. + 3) at a time:

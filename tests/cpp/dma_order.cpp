@@ -16,7 +16,7 @@ using namespace ifd;
 
 template <class Kernel, class Args>
 static void run(const char* name, int MT, int units, int waves, int groups, Kernel k, Args a, std::vector<float>& C) {
-  emu::units = units, emu::bad = 0;
+  emu::units = units, emu::unread = units / 3 * 3, emu::bad = 0;  // three register sets
   gridDim.x = 1, blockIdx.x = 0;
   long nan = 0;
   for (int t = 0; t < 64 * waves; t++) {

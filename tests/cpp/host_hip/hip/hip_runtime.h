@@ -1,7 +1,8 @@
 // A stand-in for the HIP headers that lets dma_order.cpp run one lane of one wave of a kernel on the host, with its
 // loads in flight as late as its waits allow. A wave's vector-memory operations retire in issue order: a direct
 // global -> LDS load makes its bytes poison when it is issued and lands when a counted wait (or a younger operation's)
-// covers it; a load to registers only takes its place in the order.
+// covers it; a load to registers only takes its place in the order, and not even that where nothing reads what it loads (the
+// compiler may drop it): past a segment's last whole turn of the register sets.
 #pragma once
 #include <math.h>
 #include <stddef.h>
@@ -51,6 +52,7 @@ inline std::deque<Op> queue;
 inline const void* act = nullptr;  // the activations' address: their DMAs land as kTag | 64-group
 inline long mfma = 0, bad = 0;
 inline int per_unit = 1, units = 1, first = 0, step = 1;  // MFMAs of a unit, units of a segment, their 64-groups
+inline int unread = 1;                                    // the first unit whose register loads nothing reads
 inline void land() {
   const Op op = queue.front();
   queue.pop_front();
@@ -64,6 +66,9 @@ inline void dma(const void* base, uint8_t* lds, int bytes, uint32_t soff) {
   queue.push_back({lds, bytes, base == act ? kTag | soff / 128 : 0u});
 }
 inline int unit() { return (int)(mfma / per_unit % units); }
+inline void reg_load() {
+  if (unit() < unread) queue.push_back({});
+}
 inline void operand(const void* v) {
   uint32_t w[4];
   memcpy(w, v, 16);
@@ -91,11 +96,11 @@ inline void __builtin_amdgcn_global_load_lds(const void* g, __attribute__((addre
   emu::dma(g, (uint8_t*)l, 64 * size, 0);
 }
 inline emu_u4 __builtin_amdgcn_raw_buffer_load_b128(__amdgpu_buffer_rsrc_t, int, int, int) {
-  emu::queue.push_back({});
+  emu::reg_load();
   return emu_u4{0, 0, 0, 0};
 }
 inline uint32_t __builtin_amdgcn_raw_buffer_load_b32(__amdgpu_buffer_rsrc_t, int, int, int) {
-  emu::queue.push_back({});
+  emu::reg_load();
   return 0;
 }
 inline emu_f16 __builtin_amdgcn_mfma_f32_32x32x16_bf16(emu_bf8 a, emu_bf8 b, emu_f16 c, int, int, int) {
