@@ -289,21 +289,26 @@ __global__ __launch_bounds__(256, 1) void k_gemm_w(GemmWArgs p) {
 
   // Unit i issues the second half of A(i + RA - 1)'s DMAs (sub-step 0), W(i + RW - 1) (sub-step 1) and, after its
   // barrier, the first half of A(i + RA) (sub-step 3) into the slab whose last fragments were read in sub-step 2. The
-  // prologue leaves the streams as if unit -1 had run: W(0 .. RW - 2), A(0 .. RA - 2), half of A(RA - 1).
-#pragma unroll
-  for (int s = 0; s < RW - 1; s++) {
+  // prologue leaves the streams as if units 1 - RA .. -1 had run, in their order, so that the units' wait counts what was
+  // issued from unit 0 on: W(0 .. RW - RA - 1), then A(s) and W(RW - RA + s) for s = 0 .. RA - 2, half of A(RA - 1).
+  auto prologue_w = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
     for (int d = 0; d < 3; d++) issue_w(wring + s * kWStage, d);
     adv_w();
-  }
+  };
+#pragma unroll
+  for (int s = 0; s < RW - RA; s++) prologue_w(s);
 #pragma unroll
   for (int s = 0; s < RA; s++) {
 #pragma unroll
     for (int d = 0; d < (s + 1 < RA ? MT : HA); d++) issue_a(aring + s * AB, d);
-    if (s + 1 < RA) adv_a();
+    if (s + 1 < RA) {
+      adv_a();
+      prologue_w(RW - RA + s);
+    }
   }
-  // W(0), W(1) and A(0) have landed: the younger DMAs are A(1 .. RA - 2) and the half
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((RA - 2) * MT + HA) : "memory");
+  // W(0), W(1) and A(0) have landed: the younger DMAs are W(RW - RA .. RW - 2), A(1 .. RA - 2) and the half
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((RA - 1) * 3 + (RA - 2) * MT + HA) : "memory");
 #pragma unroll
   for (int nb = 0; nb < 2; nb++) {
     read_codes(wring, nb);
@@ -325,7 +330,8 @@ __global__ __launch_bounds__(256, 1) void k_gemm_w(GemmWArgs p) {
       if (t == 1)
 #pragma unroll
         for (int nb = 0; nb < 2; nb++) scales(nb), w3[nb] = cw[nb][3];
-      // A(i + 1) and, older, W(i + 2) have landed: younger are A(i + 2 .. i + RA - 1) and the W between them and since
+      // A(i + 1) and, older, W(i + 2) have landed: younger are A(i + 2 .. i + RA - 1) and the W of the RA - 1 units that
+      // issued them, this one included
       if (t == 3)
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((RA - 2) * (MT + 3) + 3) : "memory");
       const uint8_t* const src = aring + (asw[(t + 1) & 3] + (t == 3 ? sln : sl));

@@ -36,7 +36,7 @@ def replay(tmp_path_factory):
     return lambda kernel: subprocess.run([exe, kernel], check=True, capture_output=True, text=True).stdout.splitlines()
 
 
-@pytest.mark.parametrize("kernel,cases", [("n", 8 * 9)])
+@pytest.mark.parametrize("kernel,cases", [("n", 8 * 9), ("w", 5 * 9)])
 def test_operands_have_landed(replay, kernel, cases):
     lines = replay(kernel)
     assert len(lines) == cases
