@@ -405,7 +405,10 @@ int launch_gemm_t(const uint16_t* A, int lda, const void* wt, int N, int K, void
     if (n) return launch_gemm_n(A, lda, nullptr, 0, wt, N, K, C, ldc, M, mode, gemm_n_affine(M, N, K, mode), ws, ws_bytes, st);
     const size_t plain = gemm_t_workspace(M, N, K, 0);
     uint16_t* gu = (uint16_t*)((char*)ws + align_up(plain, 256));
-    IFD_TRY(launch_gemm_t(A, lda, wt, N, K, gu, N, M, 0, ws, plain, st));
+    // (in the SwiGLU's own arithmetic: the stream-K rule never took these widths, so up to 64 rows it is the affine one)
+    IFD_TRY(gemm_w_applies(M, N, K, 0) ? launch_gemm_w(A, lda, wt, N, K, gu, N, M, 0, ws, plain, st)
+                                       : launch_gemm_n(A, lda, nullptr, 0, wt, N, K, gu, N, M, 0,
+                                                       gemm_n_affine(M, N, K, mode), ws, plain, st));
     return launch_silu_mul(gu, N, (uint16_t*)C, ldc, N / 2, M, st);
   }
   const GtPlan pl = gemm_t_plan(M, N, K);
