@@ -276,7 +276,7 @@ int ifd_gemm_t64(const void* A, int lda, const void* wt, int N, int K, void* C, 
 // Per-group activations: [Ab = bf16(U) | sxT | the GEMM's own workspace] in the body.
 namespace {
 struct W4a8gLayout {
-  size_t ab, sxt, gemm, total;
+  size_t ab, sxt, gemm, least, total;  // least, total: with the GEMM's least and full workspace
   int Mp;
 };
 W4a8gLayout w4a8g_layout(int M, int N, int K, int mode) {
@@ -286,6 +286,7 @@ W4a8gLayout w4a8g_layout(int M, int N, int K, int mode) {
   L.sxt = align_up((size_t)M * K * 2, 256);
   L.gemm = L.sxt + align_up((size_t)(K / 64) * L.Mp * 4, 256);
   L.total = L.gemm + (M <= 16 ? qmv_t_workspace(M, N, K, mode) : gemm_t_a8_workspace(M, N, K, mode));
+  L.least = M <= 16 ? L.total : L.gemm + gemm_t_a8_least_workspace(M, N, K, mode);
   return L;
 }
 }  // namespace
@@ -309,7 +310,7 @@ int ifd_gemm_t64_w4a8(const int8_t* U, const float* XS, int per_token, const voi
   if (per_token) return launch_w4a8_t(U, XS, wt, N, K, C, ldc, M, mode, w.body, w.bytes, S(stream));
   // per (row, 64-group) scales: xq as bf16 integers through the affine T64 kernels
   const W4a8gLayout L = w4a8g_layout(M, N, K, mode);
-  if (!w.body || w.bytes < L.total)
+  if (!w.body || w.bytes < L.least)
     return fail(IFD_ERR_WORKSPACE, "gemm_t64_w4a8 needs %zu bytes of workspace, got %zu", with_header(L.total),
                 ws_bytes);
   char* b = (char*)w.body;
@@ -679,16 +680,19 @@ int ifd_moe_ffn_t64(const void* xn, int T, int H, const void* router, int E, int
 
 // ---- the dense decode MLP block -----------------------------------------------------------------------------------
 namespace {
-size_t mlp_gemm_scratch(int M, int H, int I) {
-  const size_t gu = M <= 16 ? qmv_t_workspace(M, 2 * I, H, kModeSwiglu) : gemm_t_workspace(M, 2 * I, H, kModeSwiglu);
-  const size_t dn = M <= 16 ? qmv_t_workspace(M, H, I, 1) : gemm_t_workspace(M, H, I, 1);
-  return align_up(std::max(gu, dn), 256);
+size_t mlp_gemm_scratch(int M, int H, int I, bool least) {
+  const auto ws = M <= 16 ? [](int m, int n, int k, int mode) { return qmv_t_workspace(m, n, k, mode); }
+                  : least ? gemm_t_least_workspace
+                          : gemm_t_workspace;
+  return align_up(std::max(ws(M, 2 * I, H, kModeSwiglu), ws(M, H, I, 1)), 256);
 }
+// the normed rows and the activation, behind the GEMMs' scratch
+size_t mlp_rows(int M, int H, int I) { return align_up((size_t)M * H * 2, 256) + (size_t)M * I * 2; }
 }  // namespace
 
 size_t ifd_mlp_decode_workspace(int M, int H, int I) {
   if (M <= 0 || H <= 0 || I <= 0) return 0;
-  return with_header(mlp_gemm_scratch(M, H, I) + align_up((size_t)M * H * 2, 256) + (size_t)M * I * 2);
+  return with_header(mlp_gemm_scratch(M, H, I, false) + mlp_rows(M, H, I));
 }
 
 int ifd_mlp_decode(void* x, int ldx, const void* norm_w, float eps, const void* gu_t64, const void* dn_t64, int M,
@@ -700,12 +704,13 @@ int ifd_mlp_decode(void* x, int ldx, const void* norm_w, float eps, const void* 
   if (M == 0) return IFD_OK;
   IFD_CHECK(x && norm_w && gu_t64 && dn_t64 && aligned(x, 16) && aligned(gu_t64, 16) && aligned(dn_t64, 16),
             "null or misaligned pointer");
-  const size_t need = ifd_mlp_decode_workspace(M, H, I);
+  const size_t rows = mlp_rows(M, H, I);
   const WsView w = ws_view(workspace, ws_bytes);
-  if (!workspace || ws_bytes < need || !aligned(workspace, 16))
-    return fail(IFD_ERR_WORKSPACE, "mlp_decode needs %zu bytes of 16-byte aligned workspace, got %zu", need, ws_bytes);
+  if (!workspace || ws_bytes < with_header(mlp_gemm_scratch(M, H, I, true) + rows) || !aligned(workspace, 16))
+    return fail(IFD_ERR_WORKSPACE, "mlp_decode needs %zu bytes of 16-byte aligned workspace, got %zu",
+                ifd_mlp_decode_workspace(M, H, I), ws_bytes);
   hipStream_t st = S(stream);
-  const size_t G = mlp_gemm_scratch(M, H, I);
+  const size_t G = std::min(mlp_gemm_scratch(M, H, I, false), (w.bytes - rows) / 256 * 256);
   uint16_t* xn = (uint16_t*)((char*)w.body + G);
   uint16_t* act = (uint16_t*)((char*)w.body + G + align_up((size_t)M * H * 2, 256));
   IFD_TRY(launch_rmsnorm((const uint16_t*)x, ldx, (const uint16_t*)norm_w, xn, H, M, H, eps, st));

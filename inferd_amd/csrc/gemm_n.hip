@@ -429,8 +429,8 @@ constexpr double kNSegment = 4000, kNFixup = 5000, kNBytesPerNs = 5000;
 static double n_round(int MT) { return MT == 4 ? 1650 : MT == 3 ? 1400 : MT == 2 ? 1150 : 900; }
 
 // form: 0 dequantized weights, 1 the decode GEMV's arithmetic (up to 64 rows), 2 the same on int8 rows with scales per
-// 64-group (blocks of at most 64 rows)
-static NPlan n_plan(int M, int N, int K, int form) {
+// 64-group (blocks of at most 64 rows); the pieces of shared tiles fit in part_bytes
+static NPlan n_plan(int M, int N, int K, int form, size_t part_bytes = SIZE_MAX) {
   NPlan pl{};
   pl.form = form;
   pl.MT = form == 2 ? (M > 32 ? 2 : 1) : (M + 31) / 32;
@@ -444,7 +444,7 @@ static NPlan n_plan(int M, int N, int K, int form) {
   for (int S = 0; rem && S <= std::min(cu / rem, 32); S++) {
     const int nsk = S ? rem * S : cu;
     const double share = (double)rem * R / nsk, bytes = (double)share_pieces(rem, nsk) * n_slot_bytes(pl.MT);
-    if (S == 1 || share < 1) continue;
+    if (S == 1 || share < 1 || bytes > part_bytes) continue;
     const double ns = whole + std::ceil(share) * rd + kNSegment * (nsk % rem ? 1.5 : 1) + kNFixup + 2 * bytes / kNBytesPerNs;
     if (ns < pl.ns) pl.ns = ns, pl.full = tiles - rem, pl.rem = rem, pl.nsk = nsk;
   }
@@ -493,10 +493,7 @@ int launch_gemm_n(const uint16_t* A, int lda, const float* sxT, int Mp, const vo
   if (M == 0) return IFD_OK;
   if ((size_t)M * lda * 2 >= ((size_t)1 << 31) || (size_t)(K / kGroup) * Mp * 4 >= ((size_t)1 << 31))
     return fail(IFD_ERR_UNSUPPORTED, "gemm_n: operands past 2 GiB");
-  const NPlan pl = n_plan(M, N, K, form);
-  const size_t need = gemm_n_workspace(M, N, K, form);
-  if (need > ws_bytes || (need && !ws))
-    return fail(IFD_ERR_WORKSPACE, "gemm_n needs %zu bytes of workspace, got %zu", need, ws_bytes);
+  const NPlan pl = n_plan(M, N, K, form, ws ? ws_bytes : 0);
   GemmNArgs a{A, lda, (const uint8_t*)wt, (uint32_t)t64_bytes(N, K), N, K, C, ldc, M, mode, sxT, Mp, pl.tiles_m, (float*)ws,
               N % 128 == 0 ? N / 64 : 0, pl.full, pl.rem, pl.nsk};
   if (form == 2) return pl.MT == 1 ? launch_n_cfg<1, 4, 2, 3>(a, st) : launch_n_cfg<2, 4, 2, 3>(a, st);

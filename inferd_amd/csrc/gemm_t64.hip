@@ -326,22 +326,35 @@ static bool swiglu_by_product(int M, int N, int K, int mode) {
          (gemm_w_applies(M, N, K, 0) || gemm_n_applies(M, N, K, 0));
 }
 
-size_t gemm_t_workspace(int M, int N, int K, int mode) {
+// What a fast plan's pieces take, and a SwiGLU product.
+static size_t gemm_t_full_workspace(int M, int N, int K, int mode) {
   if (swiglu_by_product(M, N, K, mode))
-    return align_up(gemm_t_workspace(M, N, K, 0), 256) + (size_t)M * N * sizeof(uint16_t);
-  const bool w = gemm_w_applies(M, N, K, mode), n = gemm_n_applies(M, N, K, mode);
-  // The size decides which requests the static scratch of ifd_gemm_t64_noalloc serves, so it is never less than a split
-  // of the last 256-row tiles (from a round of them), the stream-K kernel or the K split would need.
-  size_t least = 0;
-  if ((w || n) && tiles256_fill(M, N)) {
+    return align_up(gemm_t_full_workspace(M, N, K, 0), 256) + (size_t)M * N * sizeof(uint16_t);
+  if (gemm_w_applies(M, N, K, mode)) return gemm_w_workspace(M, N, K);
+  if (gemm_n_applies(M, N, K, mode)) return gemm_n_workspace(M, N, K, gemm_n_affine(M, N, K, mode));
+  return 0;
+}
+
+// The least that a call is served with: a split of the last 256-row tiles (from a round of them; for a pair by its product
+// the product), what a stream-K kernel would take, or the K split. Calls were always served with as much, so the kernels
+// cut their tiles to fit into it.
+size_t gemm_t_least_workspace(int M, int N, int K, int mode) {
+  if (tiles256_fill(M, N) && swiglu_by_product(M, N, K, mode)) return (size_t)M * N * sizeof(uint16_t);
+  if (tiles256_fill(M, N) && (gemm_w_applies(M, N, K, mode) || gemm_n_applies(M, N, K, mode))) {
     const long tail = (long)((M + 255) / 256) * ((t64_bands(N) + 7) / 8) % 256;
-    if (tail && tail <= 128) least = (size_t)std::min({256 / tail, 8L, K / kGroup / 4L}) * tail * 256 * 256 * 4;
-  } else {
-    least = gemm_sk_applies(M, N, K, mode) ? gemm_sk_workspace(M, N, K, mode)
-                                           : epilogue_ws_bytes(gemm_t_plan(M, N, K).S, M, N, mode);
+    const long G = K / kGroup, S = tail && tail <= 128 ? std::min({256 / tail, 8L, G / 4}) : 0;
+    if (S < 2) return 0;
+    const long gps = (G + S - 1) / S;
+    return (size_t)((G + gps - 1) / gps) * tail * 256 * 256 * sizeof(float);
   }
-  if (w) return std::max(gemm_w_workspace(M, N, K), least);
-  return n ? std::max(gemm_n_workspace(M, N, K, gemm_n_affine(M, N, K, mode)), least) : least;
+  if (gemm_sk_applies(M, N, K, mode)) return gemm_sk_workspace(M, N, K, mode);
+  return epilogue_ws_bytes(gemm_t_plan(M, N, K).S, M, N, mode);
+}
+
+// Never less than the least: the size decides which requests the static scratch of ifd_gemm_t64_noalloc serves, and the K
+// split still takes operands past 2 GiB (launch_gemm_t).
+size_t gemm_t_workspace(int M, int N, int K, int mode) {
+  return std::max(gemm_t_full_workspace(M, N, K, mode), gemm_t_least_workspace(M, N, K, mode));
 }
 
 template <int MT, int NB, bool DEQ, bool A8 = false>
@@ -365,8 +378,11 @@ static int launch_gemm_t_cfg(const GemmTArgs& p, int S, hipStream_t st) {
 // 64-row tiles at most: the affine form has no dequant to share across M tiles, and four tiles' accumulators with
 // their row scales spill registers
 static GtPlan gemm_t_a8_plan(int M, int N, int K) { return gemm_t_plan(std::min(M, 64), N, K, M); }
+size_t gemm_t_a8_least_workspace(int M, int N, int K, int mode) {
+  return epilogue_ws_bytes(gemm_t_a8_plan(M, N, K).S, M, N, mode);
+}
 size_t gemm_t_a8_workspace(int M, int N, int K, int mode) {
-  const size_t least = epilogue_ws_bytes(gemm_t_a8_plan(M, N, K).S, M, N, mode);
+  const size_t least = gemm_t_a8_least_workspace(M, N, K, mode);
   return gemm_n_a8_applies(M, N, K) ? std::max(gemm_n_workspace(M, N, K, 2), least) : least;
 }
 int launch_gemm_t_a8(const uint16_t* Ab, const float* sxT, int Mp, const void* wt, int N, int K, void* C, int ldc,
@@ -375,9 +391,10 @@ int launch_gemm_t_a8(const uint16_t* Ab, const float* sxT, int Mp, const void* w
   if (K % 128) return fail(IFD_ERR_ARG, "T64 W4A8 needs K %% 128 == 0 (K=%d)", K);
   if (mode == kModeSwiglu) return fail(IFD_ERR_UNSUPPORTED, "T64 W4A8: no SwiGLU mode");
   const GtPlan pl = gemm_t_a8_plan(M, N, K);
-  const size_t need = gemm_t_a8_workspace(M, N, K, mode);
-  if (need > ws_bytes || (need && !ws))
-    return fail(IFD_ERR_WORKSPACE, "gemm_t64_w4a8 needs %zu bytes of workspace, got %zu", need, ws_bytes);
+  const size_t least = gemm_t_a8_least_workspace(M, N, K, mode);
+  if (least > ws_bytes || (least && !ws))
+    return fail(IFD_ERR_WORKSPACE, "gemm_t64_w4a8 needs %zu bytes of workspace, got %zu",
+                gemm_t_a8_workspace(M, N, K, mode), ws_bytes);
   if (gemm_n_a8_applies(M, N, K))
     return launch_gemm_n(Ab, K, sxT, Mp, wt, N, K, C, ldc, M, mode, 2, ws, ws_bytes, st);
   GemmTArgs p{Ab, K, (const uint8_t*)wt, N, K, C, ldc, M, mode, (float*)ws, pl.gps,
@@ -398,17 +415,20 @@ int launch_gemm_t(const uint16_t* A, int lda, const void* wt, int N, int K, void
   const bool by_product = !far && swiglu_by_product(M, N, K, mode);
   const bool w = !far && gemm_w_applies(M, N, K, mode), n = !far && gemm_n_applies(M, N, K, mode);
   if (by_product || w || n) {
-    const size_t need = gemm_t_workspace(M, N, K, mode);
-    if (need > ws_bytes || (need && !ws))
-      return fail(IFD_ERR_WORKSPACE, "gemm_t64 needs %zu bytes of workspace, got %zu", need, ws_bytes);
+    const size_t full = gemm_t_full_workspace(M, N, K, mode), least = gemm_t_least_workspace(M, N, K, mode);
+    if (least > ws_bytes || (least && !ws))
+      return fail(IFD_ERR_WORKSPACE, "gemm_t64 needs %zu bytes of workspace, got %zu", gemm_t_workspace(M, N, K, mode),
+                  ws_bytes);
+    const bool affine = gemm_n_affine(M, N, K, mode);
     if (w) return launch_gemm_w(A, lda, wt, N, K, C, ldc, M, mode, ws, ws_bytes, st);
-    if (n) return launch_gemm_n(A, lda, nullptr, 0, wt, N, K, C, ldc, M, mode, gemm_n_affine(M, N, K, mode), ws, ws_bytes, st);
-    const size_t plain = gemm_t_workspace(M, N, K, 0);
-    uint16_t* gu = (uint16_t*)((char*)ws + align_up(plain, 256));
-    // (in the SwiGLU's own arithmetic: the stream-K rule never took these widths, so up to 64 rows it is the affine one)
-    IFD_TRY(gemm_w_applies(M, N, K, 0) ? launch_gemm_w(A, lda, wt, N, K, gu, N, M, 0, ws, plain, st)
-                                       : launch_gemm_n(A, lda, nullptr, 0, wt, N, K, gu, N, M, 0,
-                                                       gemm_n_affine(M, N, K, mode), ws, plain, st));
+    if (n) return launch_gemm_n(A, lda, nullptr, 0, wt, N, K, C, ldc, M, mode, affine, ws, ws_bytes, st);
+    // [the product's pieces | the product], in the SwiGLU's own arithmetic: the stream-K rule never took these widths, so
+    // up to 64 rows it is the affine one
+    const size_t product = (size_t)M * N * sizeof(uint16_t);
+    const size_t pieces = std::min(full - product, (ws_bytes - product) / 256 * 256);
+    uint16_t* gu = (uint16_t*)((char*)ws + pieces);
+    IFD_TRY(gemm_w_applies(M, N, K, 0) ? launch_gemm_w(A, lda, wt, N, K, gu, N, M, 0, ws, pieces, st)
+                                       : launch_gemm_n(A, lda, nullptr, 0, wt, N, K, gu, N, M, 0, affine, ws, pieces, st));
     return launch_silu_mul(gu, N, (uint16_t*)C, ldc, N / 2, M, st);
   }
   const GtPlan pl = gemm_t_plan(M, N, K);

@@ -544,10 +544,7 @@ int launch_gemm_w(const uint16_t* A, int lda, const void* wt, int N, int K, void
                   void* ws, size_t ws_bytes, hipStream_t st) {
   if (M == 0) return IFD_OK;
   if ((size_t)M * lda * 2 >= ((size_t)1 << 31)) return fail(IFD_ERR_UNSUPPORTED, "gemm_w: operands past 2 GiB");
-  const WPlan pl = w_plan(M, N, K, kWPartMax);
-  const size_t need = (size_t)share_pieces(pl.rem, pl.nsk) * w_slot_bytes(pl.MT);
-  if (need > ws_bytes || (need && !ws))
-    return fail(IFD_ERR_WORKSPACE, "gemm_w needs %zu bytes of workspace, got %zu", need, ws_bytes);
+  const WPlan pl = w_plan(M, N, K, ws ? std::min(ws_bytes, kWPartMax) : 0);
   GemmWArgs a{A, lda, (const uint8_t*)wt, (uint32_t)t64_bytes(N, K), N, K, C, ldc, M, mode, (float*)ws, pl.tiles_m,
               pl.tiles_n, N % 256 == 0 ? N / 64 : 0, pl.full, pl.rem, pl.nsk};
   switch (pl.MT) {

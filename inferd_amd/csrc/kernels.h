@@ -70,7 +70,10 @@ int launch_pack_t64(const uint32_t* wq, const uint16_t* s, const uint16_t* b, in
                     int E, void* out, hipStream_t st);
 size_t qmv_t_workspace(int M, int N, int K, int mode, int bits = 4);
 size_t gemm_t_workspace(int M, int N, int K, int mode);
-// Prefill GEMM on T64 weights (gemm_w.hip): M > 128, modes 0-2 and SwiGLU.
+// the least that a call is served with (gemm_t64.hip)
+size_t gemm_t_least_workspace(int M, int N, int K, int mode);
+// Prefill GEMM on T64 weights (gemm_w.hip): M > 128, modes 0-2 and SwiGLU. This launcher and the next one plan within
+// the workspace they get (gemm_w_workspace, gemm_n_workspace: what the fastest plan takes).
 bool gemm_w_applies(int M, int N, int K, int mode);
 size_t gemm_w_workspace(int M, int N, int K);
 int launch_gemm_w(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
@@ -126,6 +129,7 @@ int launch_w4a8g_prep(const int8_t* U, const float* XS, int M, int K, uint16_t* 
 int launch_qmv_t_a8(const uint16_t* Ab, const float* XS, const void* wt, int N, int K, void* C, int ldc, int M,
                     int mode, unsigned* cnt, void* ws, size_t ws_bytes, hipStream_t st);
 size_t gemm_t_a8_workspace(int M, int N, int K, int mode);
+size_t gemm_t_a8_least_workspace(int M, int N, int K, int mode);
 int launch_gemm_t_a8(const uint16_t* Ab, const float* sxT, int Mp, const void* wt, int N, int K, void* C, int ldc,
                      int M, int mode, void* ws, size_t ws_bytes, hipStream_t st);
 

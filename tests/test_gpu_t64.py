@@ -656,6 +656,83 @@ def test_gemm_t64_swiglu_ragged_halves_affine(M, N, K):
     assert np.mean(out[rows] != ref) < 0.05
 
 
+def test_gemm_t64_swiglu_by_product_workspace():
+    """A gate/up pair of ragged halves also runs in what a K split of its product takes (4 fp32 copies here; its tiles are
+    then cut elsewhere, if at all), and is refused below that. Its size is that of its product and pieces, or such a split's."""
+    g, ops = _gu(), _ops()
+    from inferd_amd._lib import IFD_ERR_WORKSPACE, IFD_OK, lib
+    L = lib()
+    M, N, K = 200, 1056, 2048
+    codes, wq, s, b = gen.qlinear(N, K, seed=M)
+    A, T = g.dev(gen.activations(M, K, seed=M + 1)), ops.pack_t64(g.qlinear(wq, s, b))
+    want = g.host(ops.silu_mul(ops.gemm_t64(A, T)))
+    need, split = L.ifd_gemm_t64_swiglu_workspace(M, N, K), 4096 + 4 * M * N * 4
+    assert split < need
+
+    def call(size):
+        ws, H = torch.zeros(need, dtype=torch.uint8, device="cuda"), torch.zeros((M, N // 2), dtype=torch.bfloat16, device="cuda")
+        rc = L.ifd_gemm_t64_swiglu(A.data_ptr(), K, T.wt.data_ptr(), N, K, H.data_ptr(), N // 2, M, ws.data_ptr(), size,
+                                   torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert not ws[size:].any(), "written past the workspace"
+        return rc, g.host(H)
+
+    assert call(split - 16)[0] == IFD_ERR_WORKSPACE
+    for size in (need, split):
+        rc, H = call(size)
+        assert rc == IFD_OK, L.ifd_last_error()
+        assert np.mean(H == want) > (0.99 if size < need else 0.999)
+    M, N, K = 178, 47680, 18432  # 187 column tiles, summed whole: the product alone
+    assert L.ifd_gemm_t64_swiglu_workspace(M, N, K) == 4096 + M * N * 2
+
+
+@pytest.mark.parametrize("entry,M,N,K,size", [
+    ("gemm", 187, 1216, 768, 0),               # no K split, no workspace
+    ("gemm", 28, 64, 14592, 0),
+    ("gemm", 257, 813, 5888, 8361736),         # 10 fp32 copies of the product
+    ("w4a8", 19, 256, 5376, 337408),           # the int8 rows as bf16 and their scales
+    ("mlp", 17, 2816, 256, 300032),            # the gate/up product, the normed rows, the activation
+])
+def test_gemm_t64_k_split_workspace_serves(entry, M, N, K, size):
+    """Calls past 16 rows run in what the K split of the product would take: the tiles are then cut to fit, or not cut, so
+    that sums differ from the full workspace's by their order only (fp32, some bf16 roundings)."""
+    g, ops = _gu(), _ops()
+    from inferd_amd._lib import IFD_ERR_WORKSPACE, IFD_OK, lib
+    L, st = lib(), torch.cuda.current_stream().cuda_stream
+    codes, wq, s, b = gen.qlinear(N * (2 if entry == "mlp" else 1), K, seed=M)
+    T, x = ops.pack_t64(g.qlinear(wq, s, b)), gen.activations(M, K, seed=M + 1)
+    A = g.dev(x)
+    if entry == "mlp":
+        D = ops.pack_t64(g.qlinear(*gen.qlinear(K, N, seed=M + 2)[1:]))
+        nw = torch.ones(K, dtype=torch.bfloat16, device="cuda")
+    if entry == "w4a8":
+        U, XS = (g.dev(v) for v in orc.a8_quant(x, False))
+    full = {"gemm": L.ifd_gemm_t64_workspace, "w4a8": L.ifd_gemm_t64_w4a8_workspace,
+            "mlp": lambda m, n, k: L.ifd_mlp_decode_workspace(m, k, n)}[entry](M, N, K)
+    assert size < full
+
+    def call(size):
+        ws = torch.zeros(full, dtype=torch.uint8, device="cuda")
+        p = ws.data_ptr() if size else None
+        C = A.clone() if entry == "mlp" else torch.zeros((M, N), dtype=torch.bfloat16, device="cuda")
+        if entry == "gemm":
+            rc = L.ifd_gemm_t64(A.data_ptr(), K, T.wt.data_ptr(), N, K, C.data_ptr(), N, M, 0, p, size, st)
+        elif entry == "w4a8":
+            rc = L.ifd_gemm_t64_w4a8(U.data_ptr(), XS.data_ptr(), 0, T.wt.data_ptr(), N, K, C.data_ptr(), N, M, 0, p, size, st)
+        else:
+            rc = L.ifd_mlp_decode(C.data_ptr(), K, nw.data_ptr(), 1e-6, T.wt.data_ptr(), D.wt.data_ptr(), M, K, N, p, size, st)
+        torch.cuda.synchronize()
+        assert not ws[size:].any(), "written past the workspace"
+        return rc, g.host(C)
+
+    (rc0, want), (rc, got) = call(full), call(size)
+    assert (rc0, rc) == (IFD_OK, IFD_OK), L.ifd_last_error()
+    w, o = gen.bf16_to_f32(want), gen.bf16_to_f32(got)
+    assert np.linalg.norm(o - w) <= (4e-3 if entry == "mlp" else 1e-3) * np.linalg.norm(w) and o.any()
+    if size:
+        assert call(size - 256)[0] == IFD_ERR_WORKSPACE
+
+
 # ---- the dense decode MLP block -----------------------------------------------------------------------------------
 @pytest.mark.parametrize("M", [1, 8, 32, 128])
 def test_mlp_decode_matches_its_sequence_at_config1(M):
