@@ -409,6 +409,8 @@ int launch_gemm_t(const uint16_t* A, int lda, const void* wt, int N, int K, void
                   void* ws, size_t ws_bytes, hipStream_t st) {
   if (M == 0) return IFD_OK;
   if (K % 128) return fail(IFD_ERR_ARG, "T64 GEMM needs K %% 128 == 0 (K=%d)", K);
+  if (tiles256_fill(M, N) && t64_bytes(N, K) >= ((size_t)1 << 31))
+    return fail(IFD_ERR_UNSUPPORTED, "gemm_t64: %zu bytes of weights past 2 GiB at a round of 256 x 256 tiles", t64_bytes(N, K));
   // activations past a buffer's 2 GiB (a large row stride): the K split, which addresses them by pointer, takes them
   // at shapes below the stream-K rule, as it always has; gemm_w.hip and gemm_n.hip refuse them
   const bool far = (size_t)M * lda * 2 >= ((size_t)1 << 31) && !tiles256_fill(M, N) && !gemm_sk_applies(M, N, K, mode);

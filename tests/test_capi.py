@@ -247,3 +247,12 @@ def test_moe_rows_checks():
 def test_noalloc_scratch_serves_wide_linears(M, N, K):
     """A head over a whole vocabulary, or a wide layer, fits the static scratch of ifd_gemm_t64_noalloc."""
     assert _lib.lib().ifd_gemm_t64_workspace(M, N, K) <= 68 << 20  # IFD_NOALLOC_SCRATCH_BYTES
+
+
+def test_gemm_t64_refuses_weights_past_2gib_in_prefill_tiles():
+    """A round or more of 256 x 256 tiles with T64 weights past 2 GiB is refused before any launch, both entries."""
+    L, big = _lib.lib(), 1 << 40
+    M, N, K = 256, 262144, 16384
+    assert L.ifd_t64_bytes(N, K, 1) >= 1 << 31
+    assert L.ifd_gemm_t64(4096, K, 4096, N, K, 4096, N, M, 0, 4096, big, None) == _lib.IFD_ERR_UNSUPPORTED
+    assert L.ifd_gemm_t64_swiglu(4096, K, 4096, N, K, 4096, N // 2, M, 4096, big, None) == _lib.IFD_ERR_UNSUPPORTED
