@@ -534,6 +534,15 @@ def test_gemm_t64_swiglu_prefill_tiles():
     assert np.array_equal(g.host(ops.gemm_t64_swiglu(A, T)), g.host(ops.silu_mul(ops.gemm_t64(A, T))))
 
 
+def _lane_rows(M):
+    """Rows of every residue modulo 32 (a row's place among a wave's lanes and a lane's sums), spread over the row tiles,
+    with the last two."""
+    tiles = (M + 31) // 32
+    rows = {32 * (r % tiles) + r for r in range(32)} | {r for r in range(32)} | {M - 2, M - 1}
+    rows = {r if r < M else r - 32 for r in rows}
+    return np.array(sorted(r for r in rows if 0 <= r < M))
+
+
 @pytest.mark.parametrize("M,N,K,mode,off", [
     (129, 1024, 1024, 0, 0),    # one tile of 160 rows, 31 of them past M; every tile shared by several blocks
     (160, 1040, 1024, 1, 0),    # whole 160-row tiles; the last band is half past N (16-byte stores stop there)
@@ -565,10 +574,10 @@ def test_gemm_t64_prefill(M, N, K, mode, off):
     assert np.array_equal(outs[0], outs[1])
     if mode != 2:
         assert np.array_equal(outs[0][:, :off], C0[:, :off]), "stores outside the columns"
-    rows = np.unique(np.r_[np.linspace(0, M - 1, 9).astype(int), M - 2])
+    rows = _lane_rows(M)
     Y = orc.qmm(np.ascontiguousarray(A[rows]), wq, s, b)
     ref = Y + gen.bf16_to_f32(C0[rows][:, off:]) if mode == 1 else Y
-    gen.check_out(outs[0][rows][:, off:], ref, 1e-2, (M, N, K, mode, off), fp32=mode == 2)
+    gen.check_out(outs[0][rows][:, off:], ref, 1e-4 if mode == 2 else 1e-2, (M, N, K, mode, off), fp32=mode == 2)
 
 
 @pytest.mark.parametrize("M,N,K", [(300, 17408, 1024), (777, 9216, 512), (1025, 16384, 256)])
@@ -595,7 +604,7 @@ def test_gemm_t64_w4a8_per_group_batches(M, N, K, mode):
     outs = [g.host(ops.gemm_t64_w4a8(g.dev(U), g.dev(XS), T, g.dev(C0) if mode == 1 else None, mode=mode,
                                      per_token=False)) for _ in range(2)]
     assert np.array_equal(outs[0], outs[1])
-    rows = np.unique(np.r_[np.linspace(0, M - 1, 9).astype(int), M - 2])
+    rows = _lane_rows(M)
     Y = orc.w4a8(np.ascontiguousarray(U[rows]), np.ascontiguousarray(XS[rows]), wq, s, b)
     ref = Y + gen.bf16_to_f32(C0[rows]) if mode == 1 else Y
     gen.check_out(outs[0][rows], ref, 1e-4 if mode == 2 else 1e-2, (M, N, K, mode), fp32=mode == 2)
@@ -624,10 +633,10 @@ def test_gemm_t64_decode_batches(M, N, K, mode):
     C0 = gen.activations(M, N, seed=M + 4)
     outs = [g.host(ops.gemm_t64(g.dev(A), T, g.dev(C0) if mode == 1 else None, mode=mode)) for _ in range(2)]
     assert np.array_equal(outs[0], outs[1])
-    rows = np.unique(np.r_[np.linspace(0, M - 1, 9).astype(int), M - 2])
+    rows = _lane_rows(M)
     Y = _t64_arith(M, N, K)(np.ascontiguousarray(A[rows]), wq, s, b)
     ref = Y + gen.bf16_to_f32(C0[rows]) if mode == 1 else Y
-    gen.check_out(outs[0][rows], ref, 1e-2, (M, N, K, mode), fp32=mode == 2)
+    gen.check_out(outs[0][rows], ref, 1e-4 if mode == 2 else 1e-2, (M, N, K, mode), fp32=mode == 2)
 
 
 @pytest.mark.parametrize("M,N,K", [(20, 1056, 512), (100, 34816, 256), (100, 1056, 512), (200, 1056, 512)])
@@ -639,6 +648,21 @@ def test_gemm_t64_swiglu_past_16_rows(M, N, K):
     A = g.dev(gen.activations(M, K, seed=M + 1))
     T = ops.pack_t64(g.qlinear(wq, s, b))
     assert np.array_equal(g.host(ops.gemm_t64_swiglu(A, T)), g.host(ops.silu_mul(ops.gemm_t64(A, T))))
+
+
+@pytest.mark.parametrize("M,N,K", [(48, 33024, 512), (48, 1024, 768), (80, 33024, 512), (80, 1024, 1280), (128, 33024, 256)])
+def test_gemm_t64_swiglu_decode_batches(M, N, K):
+    """The fused gate/up pair of 33 to 128 rows (tiles of 64, 96 and 128 rows, whole and shared) against the oracle's SwiGLU
+    of its bf16 product: sums in another order move a gate or up by a bf16 step in less than 1% of the places."""
+    g, ops = _gu(), _ops()
+    codes, wq, s, b = gen.qlinear(N, K, seed=M + N)
+    A = gen.activations(M, K, seed=M + 1)
+    rows = _lane_rows(M)
+    out = g.host(ops.gemm_t64_swiglu(g.dev(A), ops.pack_t64(g.qlinear(wq, s, b))))[rows]
+    ref = orc.silu_mul(gen.f32_to_bf16(_t64_arith(M, N, K)(np.ascontiguousarray(A[rows]), wq, s, b)))
+    h, hr = gen.bf16_to_f32(out), gen.bf16_to_f32(ref)
+    assert np.mean(out != ref) < 0.02
+    assert np.linalg.norm(h - hr) < 1e-3 * np.linalg.norm(hr)
 
 
 @pytest.mark.parametrize("M,N,K", [(24, 22000, 256), (64, 22000, 512)])
