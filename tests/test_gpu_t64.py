@@ -680,6 +680,33 @@ def test_gemm_t64_swiglu_ragged_halves_affine(M, N, K):
     assert np.mean(out[rows] != ref) < 0.05
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 1024, 1024), (40, 1056, 2048), (200, 1024, 1024)])
+def test_gemm_t64_far_rows(M, N, K):
+    """Rows further apart than 2 GiB of activations allow, at few column tiles: the K split, which addresses them by pointer
+    (32-, 64- and 128-row tiles), plain and with the SwiGLU; where the stream-K rule holds they are refused."""
+    g, ops = _gu(), _ops()
+    from inferd_amd._lib import IFD_ERR_UNSUPPORTED, IFD_OK, lib
+    L, st = lib(), torch.cuda.current_stream().cuda_stream
+    lda = ((1 << 31) // (2 * M) + 8) // 8 * 8
+    codes, wq, s, b = gen.qlinear(N, K, seed=M + N)
+    T = ops.pack_t64(g.qlinear(wq, s, b))
+    x = gen.activations(M, K, seed=M + 1)
+    A = torch.empty((M - 1) * lda + K, dtype=torch.bfloat16, device="cuda").as_strided((M, K), (lda, 1))
+    A.copy_(g.dev(x))
+    C, H = (torch.zeros((M, n), dtype=d, device="cuda") for n, d in ((N, torch.float32), (N // 2, torch.bfloat16)))
+    ws = torch.zeros(max(L.ifd_gemm_t64_workspace(M, N, K), L.ifd_gemm_t64_swiglu_workspace(M, N, K)), dtype=torch.uint8,
+                     device="cuda")
+    assert L.ifd_gemm_t64(A.data_ptr(), lda, T.wt.data_ptr(), N, K, C.data_ptr(), N, M, 2, ws.data_ptr(), ws.numel(), st) == IFD_OK
+    assert L.ifd_gemm_t64_swiglu(A.data_ptr(), lda, T.wt.data_ptr(), N, K, H.data_ptr(), N // 2, M, ws.data_ptr(), ws.numel(),
+                                 st) == IFD_OK
+    Y = _t64_arith(M, N, K)(x, wq, s, b)
+    gen.check_f32(g.host(C), Y, 1e-4, (M, N, K))
+    assert np.mean(g.host(H) != orc.silu_mul(gen.f32_to_bf16(Y))) < 0.02
+    far = (1 << 31) // (2 * 65) // 8 * 8 + 8
+    assert L.ifd_gemm_t64(A.data_ptr(), far, T.wt.data_ptr(), N, K, C.data_ptr(), N, 65, 2, ws.data_ptr(), 1 << 40,
+                          st) == IFD_ERR_UNSUPPORTED
+
+
 def test_gemm_t64_swiglu_by_product_workspace():
     """A gate/up pair of ragged halves also runs in what a K split of its product takes (4 fp32 copies here; its tiles are
     then cut elsewhere, if at all), and is refused below that. Its size is that of its product and pieces, or such a split's."""
