@@ -483,7 +483,9 @@ static int launch_n_cfg(const GemmNArgs& a, hipStream_t st) {
   switch (a.mode) {
     case 1: return launch_n_mode<MT, NKQ, FORM, NS, 1>(a, st);
     case 2: return launch_n_mode<MT, NKQ, FORM, NS, 2>(a, st);
-    case kModeSwiglu: return launch_n_mode<MT, NKQ, FORM, NS, kModeSwiglu>(a, st);
+    case kModeSwiglu:
+      if constexpr (FORM != 2) return launch_n_mode<MT, NKQ, FORM, NS, kModeSwiglu>(a, st);
+      return fail(IFD_ERR_UNSUPPORTED, "gemm_n: no SwiGLU on int8 rows");
     default: return launch_n_mode<MT, NKQ, FORM, NS, 0>(a, st);
   }
 }

@@ -23,9 +23,6 @@
 // is issued by a whole wave under wave-uniform control flow (the LDS base goes to M0). Finished tiles are staged
 // through LDS and leave as whole rows.
 //
-// SwiGLU mode: tile t holds gate bands 4t..4t+3 (waves 0, 1) and the matching up bands (waves 2, 3); the staged tile
-// (or the fixup) gives h = silu(bf16(gate)) * bf16(up) (reference silu_mul, core.metal:777-787).
-//
 // A band's codes are two 1 KB halves per group, dequantized from the stored q - 128 bytes to bf16(s q + b).
 #include <algorithm>
 #include <type_traits>
@@ -71,7 +68,6 @@ struct GemmSkArgs {
   float* part;  // partial slots [2 nblk][8 bands][MT * 16 / 4][64] float4 (MFMA fragment order)
   uint32_t part_bytes;
   int tiles_m, tiles_n, G, nblk;
-  int swi;  // SwiGLU mode: bands per half (N / 64); 0 otherwise
   // k_sk_fixup only: the stream-K tiles are tiles tile0 .. tile0 + ntiles - 1 of the tile order, and each output row
   // is scaled by rs[row * rs_stride] before its store (rs null: no scale)
   int tile0, ntiles;
@@ -135,8 +131,7 @@ __device__ __forceinline__ void sk_body(const GemmSkArgs& p, uint8_t* lds, const
   const int tile_first = u0 / G, tile_last = (u1 - 1) / G;
 
   auto phys_band = [&](int tn, int lb) __attribute__((always_inline)) {  // physical band of local band lb (0..7)
-    const int bb = p.swi ? (lb < 4 ? 4 * tn + lb : p.swi + 4 * tn + lb - 4) : 8 * tn + lb;
-    return min(bb, nbands - 1);
+    return min(8 * tn + lb, nbands - 1);
   };
   const __amdgpu_buffer_rsrc_t ra =
       __builtin_amdgcn_make_buffer_rsrc((void*)p.A, 0, (int)((uint32_t)p.M * p.lda * 2u), 0x00020000);
@@ -356,7 +351,7 @@ __device__ __forceinline__ void sk_body(const GemmSkArgs& p, uint8_t* lds, const
   // every DMA and partial store has landed; LDS is free once all waves are past their reads
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
-  // A tile is staged through LDS ([BM][kSkRow] fp32) and leaves as rows (SwiGLU: h). Lane (wave, j, h) stages
+  // A tile is staged through LDS ([BM][kSkRow] fp32) and leaves as rows. Lane (wave, j, h) stages
   // acc[nb][a][r] at row a 32 + 8 (r / 4) + 4 h + r % 4, column 32 (2 wave + nb) + j, which are also the entries of its
   // float4s in a piece slot. The caller has passed a barrier since the staging area was last read.
   auto stg_at = [&](int nb, int a, int r) __attribute__((always_inline)) {
@@ -373,31 +368,16 @@ __device__ __forceinline__ void sk_body(const GemmSkArgs& p, uint8_t* lds, const
   auto emit_tile = [&](int t) __attribute__((always_inline)) {
     __syncthreads();
     const int tm = t % p.tiles_m, tn = t / p.tiles_m;
-    if (p.swi) {
-      uint16_t* C = (uint16_t*)p.C;
-      for (int e = tid; e < BM * 32; e += kSkThreads) {
-        const int row = e >> 5, c4 = (e & 31) * 4, grow = tm * BM + row;
-        if (grow >= p.M) continue;
-        const float4 g = *(const float4*)(stg + row * kSkRow + c4);
-        const float4 u = *(const float4*)(stg + row * kSkRow + 128 + c4);
-        const uint32_t lo =
-            pack_bf2(swiglu_f(bf2f(f2bf(g.x)), bf2f(f2bf(u.x))), swiglu_f(bf2f(f2bf(g.y)), bf2f(f2bf(u.y))));
-        const uint32_t hi =
-            pack_bf2(swiglu_f(bf2f(f2bf(g.z)), bf2f(f2bf(u.z))), swiglu_f(bf2f(f2bf(g.w)), bf2f(f2bf(u.w))));
-        *(u32x2*)(C + (size_t)grow * p.ldc + tn * 128 + c4) = u32x2{lo, hi};
-      }
-    } else {
-      for (int e = tid; e < BM * 64; e += kSkThreads) {
-        const int row = e >> 6, c4 = (e & 63) * 4, grow = tm * BM + row, gcol = tn * 256 + c4;
-        if (grow >= p.M || gcol >= p.N) continue;
-        const float* sv = stg + row * kSkRow + c4;
-        const size_t o = (size_t)grow * p.ldc + gcol;
-        if (gcol + 4 <= p.N && (o & 3) == 0 && p.mode != 1) {
-          if (p.mode == 2) *(float4*)((float*)p.C + o) = *(const float4*)sv;
-          else *(u32x2*)((uint16_t*)p.C + o) = u32x2{pack_bf2(sv[0], sv[1]), pack_bf2(sv[2], sv[3])};
-        } else {
-          for (int k = 0; k < 4 && gcol + k < p.N; k++) store_mode(p.C, o + k, sv[k], p.mode);
-        }
+    for (int e = tid; e < BM * 64; e += kSkThreads) {
+      const int row = e >> 6, c4 = (e & 63) * 4, grow = tm * BM + row, gcol = tn * 256 + c4;
+      if (grow >= p.M || gcol >= p.N) continue;
+      const float* sv = stg + row * kSkRow + c4;
+      const size_t o = (size_t)grow * p.ldc + gcol;
+      if (gcol + 4 <= p.N && (o & 3) == 0 && p.mode != 1) {
+        if (p.mode == 2) *(float4*)((float*)p.C + o) = *(const float4*)sv;
+        else *(u32x2*)((uint16_t*)p.C + o) = u32x2{pack_bf2(sv[0], sv[1]), pack_bf2(sv[2], sv[3])};
+      } else {
+        for (int k = 0; k < 4 && gcol + k < p.N; k++) store_mode(p.C, o + k, sv[k], p.mode);
       }
     }
   };
@@ -426,8 +406,7 @@ __global__ __launch_bounds__(kSkThreads, 1) void k_gemm_sk(GemmSkArgs p) {
 }
 
 // Sum of a cut tile's pieces (partial slots, in unit order) and its store. Block (tile, w, a), wave q: the float4
-// fragment (a, q) of column band w of the tile (SwiGLU: gate band w with up band w + 4, giving h), the
-// loads of up to kFixBatch pieces in flight at once; whole tiles were stored by the GEMM kernel. blockIdx.x is the
+// fragment (a, q) of column band w of the tile, the loads of up to kFixBatch pieces in flight at once; whole tiles were stored by the GEMM kernel. blockIdx.x is the
 // tile's index among the stream-K tiles (units [tile G, tile G + G) of their U = ntiles G).
 constexpr int kFixBatch = 8;
 template <int MT>
@@ -446,10 +425,9 @@ __global__ __launch_bounds__(256) void k_sk_fixup(GemmSkArgs p) {
   // segment (slot 2 bb). With more blocks than units (sparse) some of those runs are empty and hold no piece.
   const uint32_t lo_f = (uint32_t)bf * U / nb;
   const float4* part = (const float4*)p.part;
-  const int w1 = p.swi ? w + 4 : w;  // SwiGLU: the up band's pieces, loaded beside the gate band's
-  float4 t0 = make_float4(0.f, 0.f, 0.f, 0.f), t1 = t0;
+  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
   for (int b0 = bf; b0 <= bl; b0 += kFixBatch) {
-    float4 x0[kFixBatch], x1[kFixBatch];
+    float4 x[kFixBatch];
     bool has[kFixBatch];
 #pragma unroll
     for (int k = 0; k < kFixBatch; k++) {
@@ -458,19 +436,14 @@ __global__ __launch_bounds__(256) void k_sk_fixup(GemmSkArgs p) {
       if (has[k] && p.sparse && bb > bf) has[k] = (uint32_t)(bb + 1) * U / nb > (uint32_t)bb * U / nb;
       if (has[k]) {
         const int slot = 2 * bb + (bb == bf && lo_f < tlo ? 1 : 0);
-        x0[k] = part[(((size_t)slot * 8 + w) * NE / 4 + a * 4 + q) * 64 + lane];
-        if (p.swi) x1[k] = part[(((size_t)slot * 8 + w1) * NE / 4 + a * 4 + q) * 64 + lane];
+        x[k] = part[(((size_t)slot * 8 + w) * NE / 4 + a * 4 + q) * 64 + lane];
       }
     }
 #pragma unroll
     for (int k = 0; k < kFixBatch; k++)
-      if (has[k]) {
-        t0.x += x0[k].x, t0.y += x0[k].y, t0.z += x0[k].z, t0.w += x0[k].w;
-        if (p.swi) t1.x += x1[k].x, t1.y += x1[k].y, t1.z += x1[k].z, t1.w += x1[k].w;
-      }
+      if (has[k]) v.x += x[k].x, v.y += x[k].y, v.z += x[k].z, v.w += x[k].w;
   }
   const int tm = (p.tile0 + tile) % p.tiles_m, tn = (p.tile0 + tile) / p.tiles_m;
-  const float4 v = t0;
   float vv[4] = {v.x, v.y, v.z, v.w};
   const int row0 = tm * BM + a * 32 + 8 * q + 4 * h;
   if (p.rs) {
@@ -478,21 +451,11 @@ __global__ __launch_bounds__(256) void k_sk_fixup(GemmSkArgs p) {
     for (int e = 0; e < 4; e++)
       if (row0 + e < p.M) vv[e] *= p.rs[(size_t)(row0 + e) * p.rs_stride];
   }
-  if (p.swi) {
-    const float4 u4 = t1;
-    const float uu[4] = {u4.x, u4.y, u4.z, u4.w};
-    const int col = (4 * tn + w) * 32 + j;
+  const int col = (8 * tn + w) * 32 + j;
+  if (col >= p.N) return;
 #pragma unroll
-    for (int e = 0; e < 4; e++)
-      if (row0 + e < p.M)
-        ((uint16_t*)p.C)[(size_t)(row0 + e) * p.ldc + col] = f2bf(swiglu_f(bf2f(f2bf(vv[e])), bf2f(f2bf(uu[e]))));
-  } else {
-    const int col = (8 * tn + w) * 32 + j;
-    if (col >= p.N) return;
-#pragma unroll
-    for (int e = 0; e < 4; e++)
-      if (row0 + e < p.M) store_mode(p.C, (size_t)(row0 + e) * p.ldc + col, vv[e], p.mode);
-  }
+  for (int e = 0; e < 4; e++)
+    if (row0 + e < p.M) store_mode(p.C, (size_t)(row0 + e) * p.ldc + col, vv[e], p.mode);
 }
 
 // ---- host side
@@ -514,12 +477,9 @@ static SkPlan gemm_sk_plan(int M, int N, int K, int bits = 4) {
   return pl;
 }
 
-// Shapes with tiles for at least a third of the CUs: there each tile is cut into a few pieces. With fewer tiles (long
-// K, narrow N) every tile is cut into many, and the aligned K split (gemm_t64.hip) moves fewer partial bytes; it is
-// still the faster kernel at 32-row tiles and with two or more 128-row M tiles over a long K (measured: N = 5120,
-// K = 17408, M = 32: 25.9 against 29.5 us; M = 256: 70.8 against 75.4 us). With one 128-row tile (64 < M <= 128)
-// stream-K is faster on every narrow shape measured (K = 17408: 45.9 against 47.6 us; N = K = 5120: 26.0 against
-// 31.2 us; N = 2048, K = 8192: 23.5 against 31.0 us), and both kernels compute bf16(s*q + b) there.
+// 4-bit shapes past 16 rows with tiles for at least a third of the CUs, or one 128-row tile: a stream-K kernel on
+// dequantized weights served them, the K split (gemm_t64.hip), whose arithmetic is affine up to 64 rows, the others. The
+// rule still says which arithmetic a call has, and with gemm_sk_workspace what it is served with.
 bool gemm_sk_applies(int M, int N, int K, int mode) {
   if (M <= 16 || K % kGroup || t64_bytes(N, K) >= ((size_t)1 << 31)) return false;
   if (mode == kModeSwiglu && N % 256) return false;
@@ -548,7 +508,7 @@ static int launch_sk_cfg(const GemmSkArgs& a, bool fixup, hipStream_t st) {
   hipLaunchKernelGGL((k_gemm_sk<MT>), dim3(a.nblk), dim3(kSkThreads), lds, st, a);
   IFD_TRY(check_launch("gemm_sk"));
   if (!fixup) return IFD_OK;
-  hipLaunchKernelGGL(k_sk_fixup<MT>, dim3(a.ntiles, a.swi ? 4 : 8, MT), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(k_sk_fixup<MT>, dim3(a.ntiles, 8, MT), dim3(256), 0, st, a);
   return check_launch("gemm_sk fixup");
 }
 
@@ -580,7 +540,7 @@ static int launch_sk(const uint16_t* A, int lda, const void* wt, int N, int K, v
   for (long t = 0; t < tiles && !fixup; t++)
     fixup = sk_block_of(t * pl.G + pl.G - 1, pl.nblk, U) != sk_block_of(t * pl.G, pl.nblk, U);
   GemmSkArgs a{A, lda, (const uint8_t*)wt, (uint32_t)wbytes, N, K, C, ldc, M, mode, (float*)ws, (uint32_t)need,
-               pl.tiles_m, pl.tiles_n, pl.G, pl.nblk, mode == kModeSwiglu ? N / 64 : 0, 0, (int)tiles, nullptr, 0, 0};
+               pl.tiles_m, pl.tiles_n, pl.G, pl.nblk, 0, (int)tiles, nullptr, 0, 0};
   if (pl.MT == 1) return launch_sk_cfg<1>(a, fixup, st);
   if (pl.MT == 2) return launch_sk_cfg<2>(a, fixup, st);
   return launch_sk_cfg<4>(a, fixup, st);
@@ -589,8 +549,8 @@ static int launch_sk(const uint16_t* A, int lda, const void* wt, int N, int K, v
 int launch_gemm_sk8(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
                     void* ws, size_t ws_bytes, hipStream_t st) {
   if (M == 0) return IFD_OK;
-  if (K % kGroup || (mode == kModeSwiglu && N % 256))
-    return fail(IFD_ERR_UNSUPPORTED, "gemm_sk8: shape N=%d K=%d", N, K);
+  if (K % kGroup || mode == kModeSwiglu)
+    return fail(IFD_ERR_UNSUPPORTED, "gemm_sk8: N=%d K=%d mode=%d", N, K, mode);
   return launch_sk(A, lda, wt, N, K, C, ldc, M, mode, ws, ws_bytes, st);
 }
 
