@@ -14,20 +14,23 @@
 //   read 50 MB of fp32 pieces at M = 128, half of the call's time. With 4 bands 256 tiles are summed whole and only the
 //   other 16 are shared out (k_gemm_n_fixup adds their pieces in K order).
 // - The weights go straight to registers, two units ahead (no other wave needs them), so that LDS holds RA activation
-//   slabs per K-group.
+//   slabs per K-group. Not so in FORM 2: the compiler takes the LDS read of the row scales for dependent on every DMA in
+//   flight and waits for all loads before it, once per unit.
 // FORM 0: weights dequantized to bf16(s q + b) (MLX qmm rounding, quantized.h:528-535), in place, one sub-step behind
 // the MFMAs. FORM 1: the decode GEMV's arithmetic (core.metal:85-171): 128 + q as exact bf16, and per 64-group the fp32
 // epilogue adds s P + (b - 128 s) X, X from an MFMA against ones. FORM 2: the reference's W4A8 with per-(row, 64-group)
 // int8 activations (w4a8.metal:24-98): A holds the codes xq as exact bf16 integers, so P = sum (128 + q) xq and
 // X = sum xq are exact (integers below 2^24), and the epilogue adds sx (s P + (b - 128 s) X) with the row's scale for
 // that group; more than 64 rows are blocks of 64, neighbours in the tile order.
-// What bounds it: at 128 rows the power-limited MFMA rate (1.65 us per round of 4 units, 1.3 PFLOP/s) and about 12 us of
-// first loads, sums and stores; below, the weight stream (0.9 us per round at 32 rows for 0.8 at 6 TB/s). Measured,
-// whole call, same box, before (stream-K or K-split tiles) -> after: 32768 x 5120 at M = 128 / 64 / 32 58.2 / 40.7 /
-// 33.1 -> 45.1 / 32.1 / 25.4 us; gate and up with SwiGLU, 34816 x 5120 (16 shared tiles), 62.5 / 43.0 / 36.0 -> 59.8 /
-// 41.6 / 32.4; 5120 x 17408 42.9 / 32.0 / 25.8 -> 37.4 / 27.2 / 20.3; 34 drawn shapes 1.05 to 1.86 times, 1.36 in the mean.
-// FORM 2 (with its prep), before the K-split tiles: 34816 x 5120 at M = 24 / 64 / 128 / 255 53.8 / 86.3 / 123.6 / 215.8 ->
-// 38.7 / 51.0 / 84.9 / 154.3 us; 5120 x 17408 at M = 24 27.8 -> 26.8.
+// What bounds it: at 128 rows rounds at 1.65 us per 4 units (1.3 PFLOP/s, the clock that the matrix cores hold under load)
+// and about 12 us of first loads, sums and stores, so that the matrix cores are busy for half of the kernel's cycles; below,
+// the weight stream (0.9 us per round at 32 rows for 0.8 at 6 TB/s) and the same 12 us. A tile change pays a memory latency:
+// the compiler waits for all loads before the first LDS write of the sums, so open_w's loads do not run on over them.
+// Measured, whole call on weights from memory, same box, before (stream-K or K-split tiles) -> after: 32768 x 5120 at M =
+// 128 / 64 / 32 62.9 / 40.2 / 31.4 -> 51.9 / 31.2 / 24.6 us; gate and up with SwiGLU, 34816 x 5120 (16 shared tiles), 61.1 /
+// 42.5 / 35.5 -> 56.4 / 39.7 / 31.2; 5120 x 17408 41.2 / 34.0 / 25.2 -> 37.5 / 29.1 / 20.7. FORM 2 (with its prep), before
+// the K-split tiles: 34816 x 5120 at M = 24 / 64 / 128 / 255 55.8 / 89.5 / 127.4 / 215.5 -> 39.7 / 52.5 / 87.1 / 158.9 us;
+// 5120 x 17408 at M = 24 28.1 -> 26.5.
 // Deeper register sets (NS 5 to 7) measured slower at 32 and 64 rows.
 // Activation slabs: [32 MT][64 bf16], 16-byte columns XOR-swizzled by row pair, filled by direct global -> LDS DMA, each
 // issued by a whole wave under wave-uniform control flow (the LDS base goes to M0).
@@ -164,7 +167,8 @@ __global__ __launch_bounds__(128 * NKQ, 1) void k_gemm_n(GemmNArgs p) {
     }
   };
   // NS units' weights, loaded NS - 1 units ahead. The stream walks the K-group's units r0 .. r0 + nr - 1 of a segment and
-  // then stays on the last one; open_w starts it on a segment, before the one before has stored its sums.
+  // then stays on the last one; open_w starts it on a segment, before the one before has stored its sums (after which the
+  // compiler waits for these loads: see above).
   u32x4 cw[NS][2];
   uint32_t csb[NS][2], vw[2], w_so;
   int w_left;

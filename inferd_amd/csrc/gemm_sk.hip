@@ -406,7 +406,8 @@ __global__ __launch_bounds__(kSkThreads, 1) void k_gemm_sk(GemmSkArgs p) {
 }
 
 // Sum of a cut tile's pieces (partial slots, in unit order) and its store. Block (tile, w, a), wave q: the float4
-// fragment (a, q) of column band w of the tile, the loads of up to kFixBatch pieces in flight at once; whole tiles were stored by the GEMM kernel. blockIdx.x is the
+// fragment (a, q) of column band w of the tile, the loads of up to kFixBatch pieces in flight at once; whole tiles were
+// stored by the GEMM kernel. blockIdx.x is the
 // tile's index among the stream-K tiles (units [tile G, tile G + G) of their U = ntiles G).
 constexpr int kFixBatch = 8;
 template <int MT>

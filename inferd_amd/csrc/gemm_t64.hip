@@ -1,6 +1,8 @@
-// GEMM on T64 weights for any M (decode batches above 16 rows and prefill): C (mode) = A . W^T.
+// GEMM on T64 weights past 16 rows: C (mode) = A . W^T. launch_gemm_t chooses the kernel: gemm_n.hip up to 128 rows,
+// gemm_w.hip past them, and the K split below (k_gemm_t) for what these do not address (weights past 2 GiB at few column
+// tiles, or rows that span more than 2 GiB of activations).
 //
-// Replaces the reference's MLX affine_qmm_t_nax (third_party/mlx/.../quantized_nax.h:938-1076, 1206-1267) and its
+// k_gemm_t replaces the reference's MLX affine_qmm_t_nax (third_party/mlx/.../quantized_nax.h:938-1076, 1206-1267) and its
 // split-K variant (engine/kernels/qmm_splitk.metal:14-107) for T64-packed weights.
 //
 // Block: 8 waves, two per SIMD; block tile BM = 32 MT rows x NBB = 4 NB bands (128 NB columns); grid x = tiles
@@ -410,7 +412,7 @@ int launch_gemm_t(const uint16_t* A, int lda, const void* wt, int N, int K, void
   if (M == 0) return IFD_OK;
   if (K % 128) return fail(IFD_ERR_ARG, "T64 GEMM needs K %% 128 == 0 (K=%d)", K);
   if (tiles256_fill(M, N) && t64_bytes(N, K) >= ((size_t)1 << 31))
-    return fail(IFD_ERR_UNSUPPORTED, "gemm_t64: %zu bytes of weights past 2 GiB at a round of 256 x 256 tiles", t64_bytes(N, K));
+    return fail(IFD_ERR_UNSUPPORTED, "gemm_t64: weights past 2 GiB (N=%d K=%d)", N, K);
   // activations past a buffer's 2 GiB (a large row stride): the K split, which addresses them by pointer, takes them
   // at shapes below the stream-K rule, as it always has; gemm_w.hip and gemm_n.hip refuse them
   const bool far = (size_t)M * lda * 2 >= ((size_t)1 << 31) && !tiles256_fill(M, N) && !gemm_sk_applies(M, N, K, mode);

@@ -26,9 +26,10 @@
 // Columns: where N % 256 == 0 a tile is bands 4 t .. + 3 of the left half of the columns and the same bands of the
 // right half, wave w owning one of each, for the plain modes too: the SwiGLU mode pairs gate and up in one lane, and
 // both modes cut the same columns at the same K, so the fused call gives the bits of the two calls it replaces.
-// Measured (whole call, same box, before -> after): 4096 x 17408 x 5120 630-650 -> 575-590 us; gate and up with SwiGLU,
-// 777 x 34816 x 5120, 350 -> 275 us (the product is not stored any more); 2048 x 5120 x 5120 133 -> 99 us; drawn shapes
-// of 129 to 1500 rows 1.02 to 1.6 times faster, 1.22 times in the mean.
+// Measured (whole call, both on one box, before -> after): 4096 x 17408 x 5120 626 -> 573 us (other boxes 647 -> 590, 664 ->
+// 614); gate and up with SwiGLU, 777 x 34816 x 5120, 341 -> 267 us (the product is not stored any more); 2048 x 5120 x 5120
+// 132 -> 101 us; drawn shapes of 129 to 1500 rows 1.02 to 1.6 times faster. The matrix cores are busy for 70% of the cycles
+// at MT = 8 and 55% at MT = 5 (counters).
 // LDS: kWRA activation slabs [32 MT][64 bf16] (16-byte columns XOR-swizzled by row pair) and kWRW weight stages (8 code
 // tiles, 8 (s, b) rows), filled by direct global -> LDS DMA; every DMA is issued by a whole wave under wave-uniform
 // control flow (the LDS base goes to M0).

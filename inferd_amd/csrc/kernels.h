@@ -88,7 +88,7 @@ int launch_gemm_n(const uint16_t* A, int lda, const float* sxT, int Mp, const vo
 int launch_gemm_t(const uint16_t* A, int lda, const void* wt, int N, int K, void* C, int ldc, int M, int mode,
                   void* ws, size_t ws_bytes, hipStream_t st);
 // The stream-K plan (gemm_sk.hip) of a 4-bit shape: whether it has tiles for a third of the CUs (or one 128-row tile),
-// and its workspace, which decode batches still report (their callers' buffers have that size).
+// and its workspace, which such calls report at least and are served with.
 bool gemm_sk_applies(int M, int N, int K, int mode);
 size_t gemm_sk_workspace(int M, int N, int K, int mode);
 // The fixup of a 128-row-tile stream-K split (gemm_sk.hip): sums the pieces of the cut tiles among the stream-K

@@ -734,7 +734,9 @@ __device__ __forceinline__ void gv_role(const GqArgs& p, uint8_t* lds, const int
   int ncut = 0, cut0 = 0, cut1 = 0;
 
   // One group pair: its weights in set S. The barrier makes its chunk visible (each gathering wave first waits for its
-  // own DMAs of it: younger are those of NA - 2 pairs and their weights) and frees the chunk before.
+  // own DMAs of it: younger are those of NA - 2 pairs and their weights) and frees the chunk before. (Where the compiler
+  // drops the last pairs' weight loads, which nothing reads, the count is too high by theirs; the pair before has then
+  // waited for its own weights, loaded after this chunk's DMA.)
   auto pair = [&](auto SC) __attribute__((always_inline)) {
     constexpr int S = decltype(SC)::value;
     if constexpr (AW) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(4 + (NA - 2) * (D + 4)) : "memory");

@@ -12,8 +12,8 @@
 #include "host.h"
 #include "kernels.h"
 
-// The largest workspace ifd_gemm_t64 asks for at decode sizes (stream-K partial slots at 65..128 rows: 64 MiB plus
-// the 4 KiB header) and at BASELINE's prefill shape; larger requests are rejected.
+// The largest workspace ifd_gemm_t64 reports at decode sizes (64 MiB plus the 4 KiB header at 65..128 rows) and for a
+// prompt of 4096 rows through 5120 x 17408; larger requests are rejected.
 constexpr size_t kNoAllocScratch = IFD_NOALLOC_SCRATCH_BYTES;
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratch];

@@ -2,7 +2,8 @@
 // blocks 0 .. n - 1 (rem < n), so that no CU waits for a partly filled last round. Block b's share starts at unit
 // share_start(b); unit u lies in the share of block share_of(u). A share is shorter than a tile, so it is part of at
 // most two, and of each it sums one piece. The pieces in order are numbered by block where every tile is cut at the
-// same units (n a multiple of rem), else by block + tile. 32-bit arithmetic: (rem G + 1) n < 2^32 (the launchers check).
+// same units (n a multiple of rem), else by block + tile. 32-bit arithmetic, (rem G + 1) n < 2^32: n is at most the CU
+// count, and with activations and weights below 2 GiB each (the launchers' bound) rem G stays below 3 million at 256 CUs.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

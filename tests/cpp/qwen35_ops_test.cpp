@@ -887,7 +887,7 @@ void test_qa8(std::mt19937& rng) {
       const bool q8 = m.qa8_route(*cs.W, M);
       BufRef dA = upload(A), dC = cs.mode == 2 ? upload(std::vector<float>((size_t)M * N)) : upload(C0);
       m.gemm(e, dA, *cs.W, dC, M, cs.mode);
-      // the plain route at 255 rows: qmm on the MLX layout; T64's stream-K or prefill tiles (qmm) at these shapes
+      // the plain route at 255 rows: qmm on the MLX layout; T64's prefill tiles (qmm) at these shapes
       auto y = q8 ? ref_wxa8(A, M, K, h.wq.data(), h.s.data(), h.b.data(), N, 4, 2) : ref_gemm(A, h, M, false);
       const std::string tag = std::string("gemm ") + cs.name + " M=" + std::to_string(M) + " mode " +
                               std::to_string(cs.mode) + (q8 ? " (QA8 route)" : " (plain route)");

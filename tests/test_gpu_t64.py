@@ -60,16 +60,15 @@ def test_gemm_t64_modes(mode):
 
 def _t64_semantics(M):
     """The T64 GEMM's arithmetic by M: the decode GEMV's exact affine form up to 16 rows (the reference's qmv/qmvt4
-    rows), bf16 dequant (MLX qmm, which the reference runs above them) beyond. The K-split fallback for shapes past
-    the counter header keeps the affine form up to 64 rows; the two forms agree well within the bar."""
+    rows), bf16 dequant (MLX qmm, which the reference runs above them) beyond. Few column tiles keep the affine form
+    up to 64 rows; the two forms agree well within the bar."""
     return orc.qmv if M <= 16 else orc.qmm
 
 
 def _t64_arith(M, N, K, cus=256):
     """The oracle form of the arithmetic ifd_gemm_t64 routes an M x [N, K] product to (capi.hip, gemm_t64.hip,
-    gemm_sk.hip): the decode GEMV's affine form (qmv4: s sum q x + b sum x) in the decode kernel (M <= 16) and in
-    the K-split kernel's 32- and 64-row tiles; bf16(s q + b) dequant (MLX qmm) in the prefill tiles, the stream-K
-    kernel and the K-split kernel's 128-row tiles."""
+    gemm_sk.hip): the decode GEMV's affine form (qmv4: s sum q x + b sum x) in the decode kernel (M <= 16) and up to
+    64 rows where there are column tiles for less than a third of the CUs; bf16(s q + b) dequant (MLX qmm) elsewhere."""
     if M <= 16:
         return orc.qmv
     bands = (N + 31) // 32
@@ -297,10 +296,10 @@ def test_gemm_t64_multi_repeats_and_matches_single_calls():
     (100, 2048, 8192, 2),   # 8 tiles of one 128-row M tile (~32 pieces each), fp32 out
 ])
 def test_gemm_t64_stream_k(M, N, K, mode):
-    """The stream-K kernel (16 < M below the prefill tiles, tiles for at least a third of the CUs, or any tile count at
-    64 < M <= 128) against the oracle on sampled rows, in every store mode, at shapes whose runs cross tile boundaries,
-    cut a tile into several or many pieces or cover whole tiles; a second call on the same workspace gives the same
-    bits (the fixup sums the pieces in unit order) and leaves the counter header zero."""
+    """Shapes with tiles for at least a third of the CUs, or of 65 to 128 rows (dequantized weights), against the oracle on
+    sampled rows, in every store mode; a second call on the same workspace gives the same bits (the fixup sums the pieces
+    in K order) and leaves the counter header zero. The pieces noted are those of a stream-K split of 256-column tiles,
+    which the shapes were chosen for."""
     from inferd_amd._lib import lib
     g, ops = _gu(), _ops()
     assert lib().ifd_gemm_t64_workspace(M, N, K) > 0
@@ -326,7 +325,7 @@ def test_gemm_t64_stream_k(M, N, K, mode):
     (1, 1024, 2048, True),     # decode kernel, K split: SwiGLU in the split-K reduction
     (4, 1024, 256, False),     # decode kernel, no split: bf16 product in the workspace, then silu_mul
     (16, 2048, 1024, True),
-    (40, 1024, 2048, True),    # stream-K kernel: SwiGLU in its fixup
+    (40, 1024, 2048, True),    # decode-batch kernel: SwiGLU in its fixup
     (40, 34816, 5120, True),
     (128, 1024, 2048, True),
     (128, 8192, 2048, True),
@@ -334,7 +333,7 @@ def test_gemm_t64_stream_k(M, N, K, mode):
 ])
 def test_gemm_t64_swiglu_matches_unfused(M, N, K, split):
     """The fused gate/up projection against gemm_t64 (mode 0) + silu_mul: the same bits from the decode and prefill
-    kernels, within one bf16 step from the stream-K kernel (whose fused tiles split K elsewhere). Against the oracle,
+    kernels, within one bf16 step between them (where the fused tiles may split K elsewhere). Against the oracle,
     as a chain: the bf16 product is within the GEMM bar, and the fused h within one bf16 step of the oracle's SwiGLU
     of that product (expf may differ in its last ulp; a product of two rounded values is no place for a max-error /
     RMS bar, whose tail a single gate rounding flip can exceed)."""
@@ -354,9 +353,8 @@ def test_gemm_t64_swiglu_matches_unfused(M, N, K, split):
         assert np.all(np.abs(h - hr) <= 2 ** -7 * np.abs(hr) + 1e-30)
         assert np.mean(h == hr) > 0.99
     else:
-        # stream-K: the fused tiles pair gate and up bands, so a column's K pieces (and the fp32 rounding of its sum)
-        # differ from the plain GEMM's. Every fused h is the SwiGLU of the unfused product with its gate and up each
-        # at most one bf16 ulp away, with one bf16 step of slack for expf's last ulp and 1e-4 RMS(h) absolute for
+        # a column's K pieces (and the fp32 rounding of its sum) may differ from the plain GEMM's. Every fused h is the
+        # SwiGLU of the unfused product with its gate and up each at most one bf16 ulp away, with one bf16 step of slack for expf's last ulp and 1e-4 RMS(h) absolute for
         # sums that cancel to far below their terms (there the fp32 summation order shows in the bf16 bits)
         hf, I = gen.bf16_to_f32(fused), N // 2
         tol = 1e-4 * np.sqrt(np.mean(gen.bf16_to_f32(unfused) ** 2))
@@ -807,8 +805,8 @@ def test_mlp_decode_matches_its_sequence_at_config1(M):
 
 @pytest.mark.parametrize("M", [1, 9, 40, 128])
 def test_mlp_decode_matches_oracle(M):
-    """x += down(SwiGLU(gate_up(rmsnorm(x)))) against the oracle's composition. At these shapes (too few column tiles
-    for the stream-K kernel) the T64 GEMMs keep the decode GEMV's affine arithmetic up to 64 rows (32- and 64-row
+    """x += down(SwiGLU(gate_up(rmsnorm(x)))) against the oracle's composition. At these shapes (few column
+    tiles) the T64 GEMMs keep the decode GEMV's affine arithmetic up to 64 rows (32- and 64-row
     tiles) and dequantize above; two chained GEMMs would compound the difference between the two forms."""
     g, ops = _gu(), _ops()
     H, I = 1024, 2048

@@ -19,8 +19,8 @@ def _noalloc(A, T, C, mode):
 
 
 def test_noalloc_matches_workspace_entry_on_consecutive_calls():
-    """Three calls in a row on the shared scratch, each smaller than the one before: a stream-K GEMM at M = 128 (64 MiB
-    of partial slots), a decode GEMV at M = 8 with the residual add (its split-K fixup counts blocks in the scratch's
+    """Three calls in a row on the shared scratch, each smaller than the one before: a GEMM at M = 128 (64 MiB of
+    reported workspace), a decode GEMV at M = 8 with the residual add (its split-K fixup counts blocks in the scratch's
     counter header, which the previous call's contents must not disturb) and M = 1 with fp32 output. Each is
     bit-identical to ifd_gemm_t64 with a workspace on the same inputs."""
     from inferd_amd import ops
