@@ -354,8 +354,9 @@ def test_gemm_t64_swiglu_matches_unfused(M, N, K, split):
         assert np.mean(h == hr) > 0.99
     else:
         # a column's K pieces (and the fp32 rounding of its sum) may differ from the plain GEMM's. Every fused h is the
-        # SwiGLU of the unfused product with its gate and up each at most one bf16 ulp away, with one bf16 step of slack for expf's last ulp and 1e-4 RMS(h) absolute for
-        # sums that cancel to far below their terms (there the fp32 summation order shows in the bf16 bits)
+        # SwiGLU of the unfused product with its gate and up each at most one bf16 ulp away, with one bf16 step of slack
+        # for expf's last ulp and 1e-4 RMS(h) absolute for sums that cancel to far below their terms (there the fp32
+        # summation order shows in the bf16 bits)
         hf, I = gen.bf16_to_f32(fused), N // 2
         tol = 1e-4 * np.sqrt(np.mean(gen.bf16_to_f32(unfused) ** 2))
         ok = np.zeros(hf.shape, dtype=bool)
